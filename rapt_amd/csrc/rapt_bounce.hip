@@ -15,20 +15,62 @@
 
 using namespace rapt;
 
-// 64-lane blocks: a run holds at most 16,384 lanes (256 waves), which 64-lane
-// blocks spread over every CU instead of a quarter of them.
+// 64-lane blocks, so that small batches spread over the CUs
 template <int M>
-static void launch_hb(rapt_ctx* c, const BounceArgs& A) {
-  const int B = 64;
-  hipLaunchKernelGGL(k_halfbounce<M>, dim3((unsigned)((A.lanes + B - 1) / B)), dim3(B), 0,
-                     c->stream, A);
+static void launch_hb(rapt_ctx* c, const BounceArgs& A, unsigned grid) {
+  hipLaunchKernelGGL(k_halfbounce<M>, dim3(grid), dim3(64), 0, c->stream, A);
 }
 
 template <int M>
-static void launch_lab(rapt_ctx* c, const BounceArgs& A, const LabelArgs& L) {
-  const int B = 64;
-  hipLaunchKernelGGL(k_bounce_labels<M>, dim3((unsigned)((A.lanes + B - 1) / B)), dim3(B), 0,
-                     c->stream, A, L);
+static void launch_lab(rapt_ctx* c, const BounceArgs& A, const LabelArgs& L, unsigned grid) {
+  hipLaunchKernelGGL(k_bounce_labels<M>, dim3(grid), dim3(64), 0, c->stream, A, L);
+}
+
+// From ORDER_MIN queries on a batch's lines are taken in k_line_order's order
+// (65,536 lines: 1.24 -> 0.82 ms, 16,384 labels 1.5 -> 1.25, its own launch 10
+// us); below, the longest line's own time is the launch's and order changes
+// nothing.
+static constexpr int64_t ORDER_MIN = 4096;
+template <int M>
+static void launch_order(rapt_ctx* c, const BounceArgs& A, bool labels, int32_t* order) {
+  hipLaunchKernelGGL(k_line_order<M>, dim3((unsigned)((A.n + ORDER_CHUNK - 1) / ORDER_CHUNK)),
+                     dim3(ORDER_THREADS), 0, c->stream, A.F, A.n, labels ? 1 : 0, A.tpos, A.Bm,
+                     order);
+}
+
+// Points a half line may hold.  A first attempt takes CAP_FIRST (a half line
+// has about 200 points at fieldlineresolution 50), with 65,536 lines resident:
+// two waves a SIMD for 2 GiB of scratch.  Only when a line overflows it is
+// the call repeated with CAP_MOST and 16,384 lines in the same memory.
+static constexpr int32_t CAP_FIRST = 512, CAP_MOST = 2048;
+
+// Fills in the resident work items, the scratch strides and the scratch
+// itself; items of five lines (groups) or one.  Returns the grid, or 0 when
+// the scratch does not fit.
+static unsigned bounce_scratch(Workspace& ws, BounceArgs& A, int64_t n, int32_t cap, bool groups,
+                               bool positions, size_t extra, char** extra_mem) {
+  const int64_t most = (int64_t)2048 * CAP_FIRST / cap;  // resident waves
+  const int64_t per_wave = groups ? GRP_PER_WAVE : 32;
+  int64_t blocks = (n + per_wave - 1) / per_wave;
+  if (blocks > most) blocks = most;
+  A.cap = cap;
+  A.slots = n < blocks * per_wave ? n : blocks * per_wave;
+  const size_t pts = (size_t)blocks * wave_bytes(cap);  // (32-bit offsets)
+  const size_t nz = positions ? (size_t)2 * cap * A.slots : 0;
+  extra = (extra + 1023) / 1024 * 1024;
+  char* mem = ws.get(extra + pts + sizeof(double) * 2 * nz);
+  if (!mem) return 0;
+  *extra_mem = mem;
+  A.pts = mem + extra;
+  A.Zs = positions ? (double*)(A.pts + pts) : nullptr;
+  A.Rs = positions ? A.Zs + nz : nullptr;
+  return (unsigned)blocks;
+}
+
+static bool any_overflow(const int32_t* status, int64_t n) {
+  for (int64_t i = 0; i < n; ++i)
+    if (status[i] == BST_OVERFLOW) return true;
+  return false;
 }
 
 // True when every one of the n values is finite (a NaN or infinite start point
@@ -39,8 +81,8 @@ static bool all_finite(const double* v, int64_t n) {
   return true;
 }
 
-// Shared host side: device copies of the inputs, the per-lane trace scratch,
-// one launch, results back.  in_w doubles in per query, out_w doubles out.
+// Shared host side: device copies of the inputs, one launch, results back.
+// in_w doubles in per query, out_w doubles out.
 static int run_bounce(rapt_ctx* c, int64_t n, const double* in, int in_w, const double* Bm,
                       double res, bool positions, const LabelArgs* lab, double* out,
                       int out_w, int32_t* status, int32_t what = 0) {
@@ -52,75 +94,71 @@ static int run_bounce(rapt_ctx* c, int64_t n, const double* in, int in_w, const 
   A.F = c->field;
   A.n = n;
   A.res = res;
-  A.cap = 2048;
   A.what = what;
-  A.lanes = n < 16384 ? n : 16384;
-  const size_t npts = (size_t)2 * A.cap * A.lanes;
-  const int narr = positions ? 6 : 4;
-  double *d_in = nullptr, *d_bm = nullptr, *d_out = nullptr, *scratch = nullptr;
-  int32_t* d_st = nullptr;
-  int rc = RAPT_OK;
-  if (hipMalloc(&d_in, sizeof(double) * in_w * n) != hipSuccess ||
-      (Bm && hipMalloc(&d_bm, sizeof(double) * n) != hipSuccess) ||
-      hipMalloc(&d_out, sizeof(double) * out_w * n) != hipSuccess ||
-      hipMalloc(&d_st, sizeof(int32_t) * n) != hipSuccess ||
-      hipMalloc(&scratch, sizeof(double) * narr * npts) != hipSuccess) {
-    rc = set_err(c, RAPT_E_OOM, "bounce scratch allocation failed");
-  } else {
+  Workspace ws(c);
+  const size_t doubles = (size_t)n * (in_w + (Bm ? 1 : 0) + out_w);
+  for (int32_t cap = CAP_FIRST;; cap = CAP_MOST) {
+    char* mem = nullptr;
+    const unsigned grid = bounce_scratch(ws, A, n, cap, lab != nullptr, positions,
+                                         sizeof(double) * doubles + sizeof(int32_t) * 2 * n, &mem);
+    if (!grid) return set_err(c, RAPT_E_OOM, "bounce scratch allocation failed");
+    double* d_in = (double*)mem;
+    double* d_bm = d_in + (size_t)in_w * n;
+    double* d_out = d_bm + (Bm ? n : 0);
+    int32_t* d_st = (int32_t*)(d_out + (size_t)out_w * n);
     A.tpos = d_in;
-    A.Bm = d_bm;
+    A.Bm = Bm ? d_bm : nullptr;
     A.out = d_out;
     A.status = d_st;
-    A.S = scratch;
-    A.Bv = scratch + npts;
-    A.Cc = scratch + 2 * npts;
-    A.Wk = scratch + 3 * npts;
-    A.Zs = positions ? scratch + 4 * npts : nullptr;
-    A.Rs = positions ? scratch + 5 * npts : nullptr;
-    if (hipMemcpyAsync(d_in, in, sizeof(double) * in_w * n, hipMemcpyHostToDevice,
-                       c->stream) != hipSuccess ||
-        (Bm && hipMemcpyAsync(d_bm, Bm, sizeof(double) * n, hipMemcpyHostToDevice,
-                              c->stream) != hipSuccess)) {
-      rc = set_err(c, RAPT_E_HIP, "bounce input copy failed");
-    } else {
+    HIP_OK(c, hipMemcpyAsync(d_in, in, sizeof(double) * in_w * n, hipMemcpyHostToDevice,
+                             c->stream));
+    if (Bm)
+      HIP_OK(c, hipMemcpyAsync(d_bm, Bm, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
+    // (a compiled user-written field would need a kernel of its own for the key)
+    A.order = nullptr;
+    if (n >= ORDER_MIN && n <= INT32_MAX && c->field.model != RAPT_FIELD_EXPR) {
+      int32_t* order = d_st + n;
       switch (c->field.model) {
-        case 1: lab ? launch_lab<1>(c, A, *lab) : launch_hb<1>(c, A); break;
-        case 2: lab ? launch_lab<2>(c, A, *lab) : launch_hb<2>(c, A); break;
-        case 5: lab ? launch_lab<5>(c, A, *lab) : launch_hb<5>(c, A); break;
-        case 8: lab ? launch_lab<8>(c, A, *lab) : launch_hb<8>(c, A); break;
-        case 9: lab ? launch_lab<9>(c, A, *lab) : launch_hb<9>(c, A); break;
-        case 10:
-          if (c->expr_mode == RAPT_EXPR_COMPILED) {  // compiled at run time
-            BounceArgs a = A;
-            LabelArgs lb = lab ? *lab : LabelArgs{};
-            void* args[] = {&a, &lb};
-            rc = rapt_jit_run_slot(c, lab ? RAPT_JIT_LABELS : RAPT_JIT_HALFBOUNCE,
-                                   (unsigned)((A.lanes + 63) / 64), 64, args);
-          } else {
-            lab ? launch_lab<10>(c, A, *lab) : launch_hb<10>(c, A);
-          }
-          break;
-        default:
-          rc = set_err(c, RAPT_E_ARG, "field-line integrals need a dipole-type, gridded or "
-                       "user-written field (model %d)", c->field.model);
+        case 1: launch_order<1>(c, A, lab != nullptr, order); break;
+        case 2: launch_order<2>(c, A, lab != nullptr, order); break;
+        case 5: launch_order<5>(c, A, lab != nullptr, order); break;
+        case 8: launch_order<8>(c, A, lab != nullptr, order); break;
+        case 9: launch_order<9>(c, A, lab != nullptr, order); break;
+        default: order = nullptr; break;
       }
-      if (rc == RAPT_OK) {
-        if (hipGetLastError() != hipSuccess ||
-            hipMemcpyAsync(out, d_out, sizeof(double) * out_w * n, hipMemcpyDeviceToHost,
-                           c->stream) != hipSuccess ||
-            hipMemcpyAsync(status, d_st, sizeof(int32_t) * n, hipMemcpyDeviceToHost,
-                           c->stream) != hipSuccess ||
-            hipStreamSynchronize(c->stream) != hipSuccess)
-          rc = set_err(c, RAPT_E_HIP, "bounce kernel failed");
-      }
+      A.order = order;
     }
+    switch (c->field.model) {
+      case 1: lab ? launch_lab<1>(c, A, *lab, grid) : launch_hb<1>(c, A, grid); break;
+      case 2: lab ? launch_lab<2>(c, A, *lab, grid) : launch_hb<2>(c, A, grid); break;
+      case 5: lab ? launch_lab<5>(c, A, *lab, grid) : launch_hb<5>(c, A, grid); break;
+      case 8: lab ? launch_lab<8>(c, A, *lab, grid) : launch_hb<8>(c, A, grid); break;
+      case 9: lab ? launch_lab<9>(c, A, *lab, grid) : launch_hb<9>(c, A, grid); break;
+      case 10:
+        if (c->expr_mode == RAPT_EXPR_COMPILED) {  // compiled at run time
+          BounceArgs a = A;
+          LabelArgs lb = lab ? *lab : LabelArgs{};
+          void* args[] = {&a, &lb};
+          const int rc =
+              rapt_jit_run_slot(c, lab ? RAPT_JIT_LABELS : RAPT_JIT_HALFBOUNCE, grid, 64, args);
+          if (rc) return rc;
+        } else {
+          lab ? launch_lab<10>(c, A, *lab, grid) : launch_hb<10>(c, A, grid);
+        }
+        break;
+      default:
+        return set_err(c, RAPT_E_ARG, "field-line integrals need a dipole-type, gridded or "
+                       "user-written field (model %d)", c->field.model);
+    }
+    if (hipGetLastError() != hipSuccess ||
+        hipMemcpyAsync(out, d_out, sizeof(double) * out_w * n, hipMemcpyDeviceToHost,
+                       c->stream) != hipSuccess ||
+        hipMemcpyAsync(status, d_st, sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream) !=
+            hipSuccess ||
+        hipStreamSynchronize(c->stream) != hipSuccess)
+      return set_err(c, RAPT_E_HIP, "bounce kernel failed");
+    if (cap == CAP_MOST || !any_overflow(status, n)) return RAPT_OK;
   }
-  (void)hipFree(d_in);
-  (void)hipFree(d_bm);
-  (void)hipFree(d_out);
-  (void)hipFree(d_st);
-  (void)hipFree(scratch);
-  return rc;
 }
 
 extern "C" int rapt_halfbounce(rapt_ctx* c, int64_t n, const double* tpos, const double* Bm,
@@ -159,10 +197,8 @@ extern "C" int rapt_bounce_labels(rapt_ctx* c, int64_t n, const double* query, d
 }
 
 template <int M>
-static void launch_bc(rapt_ctx* c, const BounceArgs& A, const BCArgs& C) {
-  const int B = 64;
-  hipLaunchKernelGGL(k_bounce_center<M>, dim3((unsigned)((A.lanes + B - 1) / B)), dim3(B), 0,
-                     c->stream, A, C);
+static void launch_bc(rapt_ctx* c, const BounceArgs& A, const BCArgs& C, unsigned grid) {
+  hipLaunchKernelGGL(k_bounce_center<M>, dim3(grid), dim3(64), 0, c->stream, A, C);
 }
 
 extern "C" int rapt_bounce_center_advance(rapt_ctx* c, int64_t n, double* tpos, const double* Bm,
@@ -197,30 +233,33 @@ extern "C" int rapt_bounce_center_advance(rapt_ctx* c, int64_t n, double* tpos, 
   A.F = c->field;
   A.n = n;
   A.res = fieldlineresolution;
-  A.cap = 2048;
-  A.lanes = n < 16384 ? n : 16384;
-  const size_t npts = (size_t)2 * A.cap * A.lanes;
-  double *d_tpos = nullptr, *d_in = nullptr, *d_rows = nullptr, *scratch = nullptr;
-  int64_t *d_nrow = nullptr, *d_off = nullptr, *d_acc = nullptr;
-  int32_t* d_st = nullptr;
-  int rc = RAPT_OK;
-  if (hipMalloc(&d_tpos, sizeof(double) * 4 * n) != hipSuccess ||
-      hipMalloc(&d_in, sizeof(double) * 4 * n) != hipSuccess ||
-      hipMalloc(&d_rows, sizeof(double) * 4 * (total > 0 ? total : 1)) != hipSuccess ||
-      hipMalloc(&d_nrow, sizeof(int64_t) * n) != hipSuccess ||
-      hipMalloc(&d_off, sizeof(int64_t) * n) != hipSuccess ||
-      hipMalloc(&d_acc, sizeof(int64_t) * n) != hipSuccess ||
-      hipMalloc(&d_st, sizeof(int32_t) * n) != hipSuccess ||
-      hipMalloc(&scratch, sizeof(double) * 4 * npts) != hipSuccess) {
-    rc = set_err(c, RAPT_E_OOM, "BounceCenter allocation failed");
-  } else {
-    A.S = scratch;
-    A.Bv = scratch + npts;
-    A.Cc = scratch + 2 * npts;
-    A.Wk = scratch + 3 * npts;
-    BCArgs C;
-    memset(&C, 0, sizeof C);
-    C.n = n;
+  BCArgs C;
+  memset(&C, 0, sizeof C);
+  C.n = n;
+  C.rtol = rtol;
+  C.atol = atol;
+  C.dstep = eyegradientstep;
+  C.nmax = nsteps > 0 ? nsteps : 500;
+  // scipy's dopri5 defaults: safety 0.9, fac1 0.2, fac2 10, beta 0 -> 0.04
+  C.c5.safe = 0.9;
+  C.c5.facc1 = 1.0 / 0.2;
+  C.c5.facc2 = 1.0 / 10.0;
+  C.c5.beta = 0.04;
+  C.c5.expo1 = 0.2 - 0.04 * 0.75;
+  Workspace ws(c);
+  const size_t rows_w = 4 * (size_t)total;
+  const size_t bytes = 8 * (8 * (size_t)n + rows_w + 3 * (size_t)n) + sizeof(int32_t) * n;
+  for (int32_t cap = CAP_FIRST;; cap = CAP_MOST) {
+    char* mem = nullptr;
+    const unsigned grid = bounce_scratch(ws, A, n, cap, true, false, bytes, &mem);
+    if (!grid) return set_err(c, RAPT_E_OOM, "BounceCenter allocation failed");
+    double* d_tpos = (double*)mem;
+    double* d_in = d_tpos + 4 * n;
+    double* d_rows = d_in + 4 * n;
+    int64_t* d_nrow = (int64_t*)(d_rows + rows_w);
+    int64_t* d_off = d_nrow + n;
+    int64_t* d_acc = d_off + n;
+    int32_t* d_st = (int32_t*)(d_acc + n);
     C.tpos = d_tpos;
     C.Bm = d_in;
     C.coef = d_in + n;
@@ -231,75 +270,54 @@ extern "C" int rapt_bounce_center_advance(rapt_ctx* c, int64_t n, double* tpos, 
     C.rows = d_rows;
     C.status = d_st;
     C.naccpt = d_acc;
-    C.rtol = rtol;
-    C.atol = atol;
-    C.dstep = eyegradientstep;
-    C.nmax = nsteps > 0 ? nsteps : 500;
-    // scipy's dopri5 defaults: safety 0.9, fac1 0.2, fac2 10, beta 0 -> 0.04
-    C.c5.safe = 0.9;
-    C.c5.facc1 = 1.0 / 0.2;
-    C.c5.facc2 = 1.0 / 10.0;
-    C.c5.beta = 0.04;
-    C.c5.expo1 = 0.2 - 0.04 * 0.75;
-    bool ok = hipMemcpyAsync(d_tpos, tpos, sizeof(double) * 4 * n, hipMemcpyHostToDevice,
-                             c->stream) == hipSuccess &&
-              hipMemcpyAsync(d_in, Bm, sizeof(double) * n, hipMemcpyHostToDevice,
-                             c->stream) == hipSuccess &&
-              hipMemcpyAsync(d_in + n, coef, sizeof(double) * n, hipMemcpyHostToDevice,
-                             c->stream) == hipSuccess &&
-              hipMemcpyAsync(d_in + 2 * n, dt, sizeof(double) * n, hipMemcpyHostToDevice,
-                             c->stream) == hipSuccess &&
-              hipMemcpyAsync(d_in + 3 * n, tcur, sizeof(double) * n, hipMemcpyHostToDevice,
-                             c->stream) == hipSuccess &&
-              hipMemcpyAsync(d_nrow, nrow, sizeof(int64_t) * n, hipMemcpyHostToDevice,
-                             c->stream) == hipSuccess &&
-              hipMemcpyAsync(d_off, off.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice,
-                             c->stream) == hipSuccess;
-    if (!ok) {
-      rc = set_err(c, RAPT_E_HIP, "BounceCenter input copy failed");
-    } else {
-      switch (c->field.model) {
-        case 1: launch_bc<1>(c, A, C); break;
-        case 2: launch_bc<2>(c, A, C); break;
-        case 8: launch_bc<8>(c, A, C); break;
-        case 10:
-          if (c->expr_mode == RAPT_EXPR_COMPILED) {
-            BounceArgs a = A;
-            BCArgs cc = C;
-            void* args[] = {&a, &cc};
-            rc = rapt_jit_run_slot(c, RAPT_JIT_BC, (unsigned)((A.lanes + 63) / 64), 64, args);
-          } else {
-            launch_bc<10>(c, A, C);
-          }
-          break;
-        default:
-          rc = set_err(c, RAPT_E_ARG, "BounceCenter needs a static dipole-type or user-written "
+    const double* in[4] = {Bm, coef, dt, tcur};
+    HIP_OK(c, hipMemcpyAsync(d_tpos, tpos, sizeof(double) * 4 * n, hipMemcpyHostToDevice,
+                             c->stream));
+    for (int k = 0; k < 4; ++k)
+      HIP_OK(c, hipMemcpyAsync(d_in + k * n, in[k], sizeof(double) * n, hipMemcpyHostToDevice,
+                               c->stream));
+    HIP_OK(c, hipMemcpyAsync(d_nrow, nrow, sizeof(int64_t) * n, hipMemcpyHostToDevice,
+                             c->stream));
+    HIP_OK(c, hipMemcpyAsync(d_off, off.data(), sizeof(int64_t) * n, hipMemcpyHostToDevice,
+                             c->stream));
+    // rows that a failed centre does not reach come back as zeros
+    if (total > 0)
+      HIP_OK(c, hipMemsetAsync(d_rows, 0, sizeof(double) * rows_w, c->stream));
+    switch (c->field.model) {
+      case 1: launch_bc<1>(c, A, C, grid); break;
+      case 2: launch_bc<2>(c, A, C, grid); break;
+      case 8: launch_bc<8>(c, A, C, grid); break;
+      case 10:
+        if (c->expr_mode == RAPT_EXPR_COMPILED) {
+          BounceArgs a = A;
+          BCArgs cc = C;
+          void* args[] = {&a, &cc};
+          const int rc = rapt_jit_run_slot(c, RAPT_JIT_BC, grid, 64, args);
+          if (rc) return rc;
+        } else {
+          launch_bc<10>(c, A, C, grid);
+        }
+        break;
+      default:
+        return set_err(c, RAPT_E_ARG, "BounceCenter needs a static dipole-type or user-written "
                        "field (model %d)", c->field.model);
-      }
-      if (rc == RAPT_OK) {
-        if (hipGetLastError() != hipSuccess ||
-            hipMemcpyAsync(tpos, d_tpos, sizeof(double) * 4 * n, hipMemcpyDeviceToHost,
-                           c->stream) != hipSuccess ||
-            (total > 0 && hipMemcpyAsync(rows, d_rows, sizeof(double) * 4 * total,
-                                         hipMemcpyDeviceToHost, c->stream) != hipSuccess) ||
-            hipMemcpyAsync(status, d_st, sizeof(int32_t) * n, hipMemcpyDeviceToHost,
-                           c->stream) != hipSuccess ||
-            hipMemcpyAsync(naccpt, d_acc, sizeof(int64_t) * n, hipMemcpyDeviceToHost,
-                           c->stream) != hipSuccess ||
-            hipStreamSynchronize(c->stream) != hipSuccess)
-          rc = set_err(c, RAPT_E_HIP, "BounceCenter kernel failed");
-      }
     }
+    if (hipGetLastError() != hipSuccess ||
+        hipMemcpyAsync(status, d_st, sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream) !=
+            hipSuccess ||
+        hipStreamSynchronize(c->stream) != hipSuccess)
+      return set_err(c, RAPT_E_HIP, "BounceCenter kernel failed");
+    if (cap != CAP_MOST && any_overflow(status, n)) continue;
+    if (hipMemcpyAsync(tpos, d_tpos, sizeof(double) * 4 * n, hipMemcpyDeviceToHost, c->stream) !=
+            hipSuccess ||
+        (total > 0 && hipMemcpyAsync(rows, d_rows, sizeof(double) * rows_w,
+                                     hipMemcpyDeviceToHost, c->stream) != hipSuccess) ||
+        hipMemcpyAsync(naccpt, d_acc, sizeof(int64_t) * n, hipMemcpyDeviceToHost, c->stream) !=
+            hipSuccess ||
+        hipStreamSynchronize(c->stream) != hipSuccess)
+      return set_err(c, RAPT_E_HIP, "BounceCenter results failed to copy");
+    return RAPT_OK;
   }
-  (void)hipFree(d_tpos);
-  (void)hipFree(d_in);
-  (void)hipFree(d_rows);
-  (void)hipFree(d_nrow);
-  (void)hipFree(d_off);
-  (void)hipFree(d_acc);
-  (void)hipFree(d_st);
-  (void)hipFree(scratch);
-  return rc;
 }
 
 template <int M>

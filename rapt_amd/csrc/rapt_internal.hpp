@@ -4,6 +4,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -64,6 +65,11 @@ struct rapt_ctx {
   // device address of this device's allocation-free scratch (the work-queue
   // and step counters of rapt_trace_device_noalloc), from hipGetSymbolAddress
   unsigned long long* noalloc_scratch = nullptr;
+  // device scratch of the field-line entry points, kept between calls
+  // (Workspace below)
+  std::mutex ws_mu;
+  void* ws = nullptr;
+  size_t ws_bytes = 0;
   std::string err;
 };
 
@@ -78,6 +84,49 @@ static inline int set_err(rapt_ctx* c, int code, const char* fmt, ...) {
     c->err = buf;
   }
   return code;
+}
+
+// The context's device scratch for the length of one entry point's call: held
+// under a lock, so calls from several threads take turns, grown when a call
+// needs more, and kept for the next call up to KEEP bytes (allocating and
+// freeing 2 GiB costs about 2 ms a call).  A call ends with its stream
+// synchronised, so nothing reads the scratch once the lock is dropped.
+struct Workspace {
+  static constexpr size_t KEEP = (size_t)5 << 29;  // 2.5 GiB
+  rapt_ctx* c;
+  std::lock_guard<std::mutex> lock;
+  explicit Workspace(rapt_ctx* ctx) : c(ctx), lock(ctx->ws_mu) {}
+  ~Workspace() {
+    if (c->ws_bytes > KEEP) drop();
+  }
+  // at least `bytes` bytes, or nullptr; what an earlier get returned is void
+  char* get(size_t bytes) {
+    if (c->ws_bytes < bytes) {
+      drop();
+      if (hipMalloc(&c->ws, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        c->ws = nullptr;
+        return nullptr;
+      }
+      c->ws_bytes = bytes;
+    }
+    return static_cast<char*>(c->ws);
+  }
+  void drop() {
+    (void)hipFree(c->ws);
+    c->ws = nullptr;
+    c->ws_bytes = 0;
+  }
+};
+// hipMalloc that takes back the kept scratch when memory runs out
+static inline hipError_t ctx_malloc(rapt_ctx* c, void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    Workspace(c).drop();
+    e = hipMalloc(p, bytes);
+  }
+  return e;
 }
 
 // run-time compiled tracer kernels of a user-written field (rapt_jit.hip)

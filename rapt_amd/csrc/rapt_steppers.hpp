@@ -370,16 +370,15 @@ constexpr double c1 = 1.157407407407407e-01, c3 = 5.489278752436647e-01,
                  c4 = 5.353313840155945e-01, c5 = -2.000000000000000e-01;
 }  // namespace rkf
 
-// One RKF45 step attempt; y1 receives the 4th-order update, returns the
-// reference's error measure max_i |r . k| / h.
+// One RKF45 step attempt from x with k0 = f(t, x); y1 receives the 4th-order
+// update, returns the reference's error measure max_i |r . k| / h.
 template <int N, class RHS>
-__device__ __forceinline__ double rkf45_attempt(RHS& f, double t, double h, const double* x,
-                                                double* y1) {
+__device__ __forceinline__ double rkf45_attempt_f0(RHS& f, double t, double h, const double* x,
+                                                   const double* k0, double* y1) {
   using namespace rkf;
   double k1[N], k2[N], k3[N], k4[N], k5[N], k6[N], tmp[N];
-  f(t, x, k1);
 #pragma unroll
-  for (int i = 0; i < N; ++i) { k1[i] *= h; tmp[i] = x[i] + b21 * k1[i]; }
+  for (int i = 0; i < N; ++i) { k1[i] = k0[i] * h; tmp[i] = x[i] + b21 * k1[i]; }
   f(t + a2 * h, tmp, k2);
 #pragma unroll
   for (int i = 0; i < N; ++i) { k2[i] *= h; tmp[i] = x[i] + b31 * k1[i] + b32 * k2[i]; }
@@ -406,10 +405,18 @@ __device__ __forceinline__ double rkf45_attempt(RHS& f, double t, double h, cons
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     k6[i] *= h;
-    r = fmax(r, __builtin_fabs(r1 * k1[i] + r3 * k3[i] + r4 * k4[i] + r5 * k5[i] + r6 * k6[i]) / h);
+    r = fmax(r, __builtin_fabs(r1 * k1[i] + r3 * k3[i] + r4 * k4[i] + r5 * k5[i] + r6 * k6[i]));
     y1[i] = x[i] + c1 * k1[i] + c3 * k3[i] + c4 * k4[i] + c5 * k5[i];
   }
-  return r;
+  return r / h;  // h > 0: the largest quotient is the largest magnitude's
+}
+
+template <int N, class RHS>
+__device__ __forceinline__ double rkf45_attempt(RHS& f, double t, double h, const double* x,
+                                                double* y1) {
+  double k0[N];
+  f(t, x, k0);
+  return rkf45_attempt_f0<N>(f, t, h, x, k0, y1);
 }
 
 }  // namespace rapt

@@ -265,6 +265,7 @@ int rapt_ctx_destroy(rapt_ctx* c) {
   (void)hipFree(c->grid_mem);
   (void)hipFree(c->grid_cells);
   (void)hipFree(c->expr_mem);
+  (void)hipFree(c->ws);
   delete c;
   return RAPT_OK;
 }
@@ -384,7 +385,7 @@ int rapt_grid_set(rapt_ctx* c, int32_t nx, int32_t ny, int32_t nz, int32_t nt, c
     }
   }
   double* mem = nullptr;
-  if (hipMalloc(&mem, sizeof(double) * total) != hipSuccess)
+  if (ctx_malloc(c, (void**)&mem, sizeof(double) * total) != hipSuccess)
     return set_err(c, RAPT_E_OOM, "grid allocation of %zu bytes failed", sizeof(double) * total);
   if (hipMemcpy(mem, h.data(), sizeof(double) * total, hipMemcpyHostToDevice) != hipSuccess) {
     (void)hipFree(mem);
@@ -696,7 +697,8 @@ int rapt_batch_set_rows(rapt_batch* b, int32_t width, const int64_t* row_cap) {
   if (tot * width != b->total_rows * b->width || !b->d_rows) {
     (void)hipFree(b->d_rows);
     b->d_rows = nullptr;
-    if (tot > 0 && hipMalloc(&b->d_rows, sizeof(double) * width * tot) != hipSuccess) {
+    if (tot > 0 &&
+        ctx_malloc(c, (void**)&b->d_rows, sizeof(double) * width * tot) != hipSuccess) {
       free(off);
       b->total_rows = 0;
       return set_err(c, RAPT_E_OOM, "trajectory buffer of %lld rows failed", (long long)tot);
@@ -1106,7 +1108,7 @@ int rapt_batch_epochs_begin(rapt_batch* b, const rapt_trace_desc* d, int32_t row
   HIP_OK(c, hipSetDevice(c->device));
   const int64_t n = b->n;
   const size_t nr = (size_t)n * rows_per_epoch;
-  bool ok = hipMalloc(&b->d_erows, sizeof(double) * nr * width) == hipSuccess &&
+  bool ok = ctx_malloc(c, (void**)&b->d_erows, sizeof(double) * nr * width) == hipSuccess &&
             hipMalloc(&b->d_eoff, sizeof(int64_t) * n) == hipSuccess &&
             hipMalloc(&b->d_ecap, sizeof(int64_t) * n) == hipSuccess &&
             hipMalloc(&b->d_left, sizeof(int32_t)) == hipSuccess &&
