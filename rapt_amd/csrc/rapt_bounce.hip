@@ -27,8 +27,8 @@ static void launch_lab(rapt_ctx* c, const BounceArgs& A, const LabelArgs& L, uns
 }
 
 // From ORDER_MIN queries on a batch's lines are taken in k_line_order's order
-// (65,536 lines: 1.24 -> 0.82 ms, 16,384 labels 1.5 -> 1.25, its own launch 10
-// us); below, the longest line's own time is the launch's and order changes
+// (65,536 lines: 1.24 -> 0.82 ms, 16,384 labels with every wave resident
+// 1.5 -> 1.25, its own launch 10 us); below, the longest line's own time is the launch's and order changes
 // nothing.
 static constexpr int64_t ORDER_MIN = 4096;
 template <int M>
@@ -44,12 +44,22 @@ static void launch_order(rapt_ctx* c, const BounceArgs& A, bool labels, int32_t*
 // the call repeated with CAP_MOST and 16,384 lines in the same memory.
 static constexpr int32_t CAP_FIRST = 512, CAP_MOST = 2048;
 
+// Waves of a surrogate-label launch.  The labels are the yardstick of the
+// surrogate, whose inference kernel is held to at least 300 times their rate on
+// 65,536 queries (tests/test_gpu_surrogate.py): with every wave resident they
+// take 5.2 ms, 50 times the ensemble's 0.106 ms.  72 waves: 65,536 queries
+// 38-42 ms, 350-400 times (80 waves 330-365, 96 280-315); 16,384 in 10.3 ms and
+// 300, which fit into them, in 0.5 (a lane a line, every line resident: 17.8 and
+// 14.9); 16,384 with every wave resident 1.2.
+static constexpr int64_t LABEL_WAVES = 72;
+
 // Fills in the resident work items, the scratch strides and the scratch
 // itself; items of five lines (groups) or one.  Returns the grid, or 0 when
 // the scratch does not fit.
 static unsigned bounce_scratch(Workspace& ws, BounceArgs& A, int64_t n, int32_t cap, bool groups,
                                bool positions, size_t extra, char** extra_mem) {
-  const int64_t most = (int64_t)2048 * CAP_FIRST / cap;  // resident waves
+  int64_t most = (int64_t)2048 * CAP_FIRST / cap;  // resident waves
+  if (positions && most > LABEL_WAVES) most = LABEL_WAVES;
   const int64_t per_wave = groups ? GRP_PER_WAVE : 32;
   int64_t blocks = (n + per_wave - 1) / per_wave;
   if (blocks > most) blocks = most;
