@@ -28,45 +28,10 @@
 #include "../../include/rapt_hip.h"
 #include "rapt_fields.hpp"
 #include "rapt_internal.hpp"
+#include "rapt_mlp.hpp"
 
 namespace rapt {
 namespace mlp {
-
-constexpr int H = 256;
-constexpr int OFF_W1 = 0;                 // [256][3]
-constexpr int OFF_B1 = OFF_W1 + H * 3;    // [256]
-constexpr int OFF_W2 = OFF_B1 + H;        // [256][256] (out, in)
-constexpr int OFF_B2 = OFF_W2 + H * H;
-constexpr int OFF_W3 = OFF_B2 + H;
-constexpr int OFF_B3 = OFF_W3 + H * H;
-constexpr int OFF_W4 = OFF_B3 + H;        // [3][256]
-constexpr int OFF_B4 = OFF_W4 + 3 * H;    // [3]
-constexpr int NPARAM = OFF_B4 + 3;        // 133,379
-constexpr int NPAD = (NPARAM + 255) / 256 * 256;
-constexpr int PACKED = 8 * 16 * 64 * 8;   // bf16 elements of one packed 256x256 layer
-
-typedef __bf16 bf16;
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-// The network is a SiLU MLP whose parameters are kept in base-2 units.  With
-// the plain network's (W1, b1, W2, b2, W3, b3, W4, b4) the stored parameters
-// are (log2(e) W1, log2(e) b1, W2, log2(e) b2, W3, log2(e) b3, ln(2) W4, b4):
-// every hidden pre-activation is then a = log2(e) z and every hidden output
-// g = log2(e) silu(z) = a / (1 + 2^-a), the same function, while the logistic
-// factor is rcp(1 + exp2(-a)), one v_exp_f32 and one v_rcp_f32 (about 1 ulp
-// each) with no scaling multiply in front.  Training and inference use these
-// same definitions, so both round the same hidden values to bf16.
-constexpr float LN2 = 0.6931471805599453f;
-__device__ __forceinline__ float sig2(float a) {
-  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-a));
-}
-__device__ __forceinline__ float act2(float a) { return a * sig2(a); }
-// d act2 / da = s (1 + ln2 a (1 - s)), s = sig2(a)
-__device__ __forceinline__ float dact2(float a) {
-  const float s = sig2(a);
-  return s * (1.0f + LN2 * a * (1.0f - s));
-}
 
 // ---- dipole baselines (the residual targets' reference point) -----------------------
 struct Base {
@@ -160,230 +125,538 @@ __device__ __forceinline__ void features(const float* q, float x[3], int side) {
 }
 
 // ---- training kernels -----------------------------------------------------------------
-// Every kernel below runs all members at once: blockIdx.z (or y) = member,
-// with per-member strides.
+// A step is two launches.  k_train_rows takes 64 samples of one member
+// through the whole network and back (everything but the weight gradients is
+// local to a sample), and leaves the four bf16 arrays that the weight
+// gradients contract over the batch, and the 64 samples' share of the small
+// gradients.  k_train_weights contracts, sums the shares and applies Adam.
+//
+// Both use v_mfma_f32_32x32x16_bf16: A operand lane l holds row l%32, K
+// indices 8(l/32)+j; B operand column l%32, K indices 8(l/32)+j; D register r
+// row 8(r/4) + 4(l/32) + r%4, column l%32.  A fragment is 64 lanes x 8 bf16 = 1
+// KB, and everything the matrix cores read from memory is stored in fragments:
+//   weights, forward:  fw[layer][out/32][in/16]:  lane out%32 + 32 (in%16/8), j in%8
+//   weights, backward: bw[layer][in/32][out/16]:  lane in%32 + 32 (out%16/8), j out%8
+//   H1, H2, dZ2, dZ3:  [sample/16][neuron/32]:    lane neuron%32 + 32 (sample%16/8), j sample%8
+// (the weight gradients' waves, a tile each, move through the samples together:
+// with the samples outside, what they read at one time is one run of memory).
+//
+// Every sum is formed in one order, whatever the launch: the MFMA chains over
+// ascending K (one chain an output, over the whole batch for the weights), 64
+// samples one after the other and then their shares, as the elementwise and
+// GEMM kernels that these two replaced did, bit for bit.
+constexpr int TB = 64;            // samples of a k_train_rows block
+constexpr int LDA = H + 8;        // row of an activation buffer in LDS (bf16), padded
+constexpr int LDF = TB + 4;       // column of the float buffer in LDS, padded
+constexpr int NSLOT_G = 10;       // shares: dW4 (3), dW1 (3), db1, db4, db3, db2
 
-// C[M][N] = op(A)[M][K] * op(B)[K][N], BF16 in, FP32 out.  op(A)[m][k] =
-// A[m*lda+k] (TA false) or A[k*lda+m]; op(B)[k][n] = B[k*ldb+n] (TB false)
-// or B[n*ldb+k].  M, N multiples of 64, K a multiple of 16.  Block: 4 waves,
-// 64 x 64 tile, wave (w/2, w%2) owns a 32 x 32 quarter.
-template <bool TA, bool TB>
-__global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, const bf16* A, int lda,
-                                              int64_t sA, const bf16* B, int ldb, int64_t sB,
-                                              float* C, int ldc, int64_t sC) {
-  __shared__ bf16 As[64][16 + 8];
-  __shared__ bf16 Bs[16][64 + 8];
-  const int mem = blockIdx.z;
-  A += mem * sA;
-  B += mem * sB;
-  C += mem * sC;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  const int t = threadIdx.x, w = t >> 6, l = t & 63;
-  const int wm = w >> 1, wn = w & 1;
-  f32x16 acc = {};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    if (!TA) {
-      const int i = t >> 2, kk = (t & 3) * 4;
-      for (int e = 0; e < 4; ++e) As[i][kk + e] = A[(int64_t)(m0 + i) * lda + k0 + kk + e];
-    } else {
-      const int kk = t >> 4, i = (t & 15) * 4;
-      for (int e = 0; e < 4; ++e) As[i + e][kk] = A[(int64_t)(k0 + kk) * lda + m0 + i + e];
+struct TrainArgs {
+  int bt;                 // samples, a multiple of 64
+  int members;
+  const int64_t* order;   // sample indices of this batch, or nullptr: rows 0 .. bt - 1
+  const float *X, *T;     // [.][3]
+  const bf16* wb;         // [members][NPAD]
+  const bf16 *fw, *bw;    // [members][2][PACKED]
+  bf16 *hp, *zp;          // [members][2][bt * H]: H1, H2 and dZ2, dZ3 fragments
+  float* part;            // [members][bt / 64][NSLOT_G][H]
+  float* Y;               // [members][bt][3] (forward alone)
+  double* loss;           // [members], or nullptr
+};
+
+// A barrier that waits for LDS alone.  __syncthreads also waits for every
+// global load and store in flight, so the weights requested for a later phase
+// and the fragments stored in an earlier one would be waited for at each phase.
+__device__ __forceinline__ void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// What is read above stays above (the scheduler sinks LDS reads to their uses)
+__device__ __forceinline__ void read_first() { asm volatile("" ::: "memory"); }
+
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+// One block of 16 waves: wave w owns samples 32 (w%2) .. + 31 and neurons 32
+// (w/2) .. + 31 of every layer.  act2' of layers 2 and 3 stays in registers
+// from the forward to the backward pass (formed with the activation, from one
+// logistic) and the activations pass through LDS as the next product's A
+// operand.  Four waves a SIMD in 128 registers: with eight waves of twice the
+// tile the same work spilled, and a barrier's wait, the output layer's chain of
+// 256 additions on three waves and the sums over 64 samples had nothing to
+// overlap with.  Loads and stores of a wave complete in order, so a load waited
+// for waits for the stores in front of it: the small parameters are in LDS from
+// the start, and what a phase stores is held until the next product's loads
+// are on their way.  4,096 samples, two members: 29 us (128 blocks), of which
+// the four products 10 and the logistics 8; with k_train_weights 48 us a step
+// against 440 us in 18 launches of elementwise kernels and 64 x 64 GEMMs.
+constexpr int RT = 1024;  // threads of a block
+template <bool TRAIN>
+__global__ __launch_bounds__(RT) void k_train_rows(TrainArgs A) {
+  __shared__ bf16 actA[TB * LDA], actB[TB * LDA];
+  __shared__ float F[H * LDF];              // [neuron][sample]: H3, later dZ1
+  __shared__ float4 xs[TB], dys[TB];
+  __shared__ float ds[3][TB], ts[3][TB];
+  __shared__ float4 w4s[3][H / 4];
+  __shared__ float w1s[3][H], bs[3][H], b4s[3];
+  const int mem = blockIdx.z, chunk = blockIdx.x, s0 = chunk * TB;
+  const int t = threadIdx.x, l = t & 63, w = t >> 6, h = l >> 5;
+  const int m = w & 1, nt = w >> 1;
+  const bf16* wb = A.wb + (int64_t)mem * NPAD;
+  // this wave's 16 fragments of a layer
+  auto tile = [&](const bf16* p, int layer) {
+    return (const bf16x8*)(p + ((int64_t)mem * 2 + layer) * PACKED) + nt * 16 * 64 + l;
+  };
+  // fragment arrays of this member: layer 0 (H1, dZ2), layer 1 (H2, dZ3)
+  bf16* hp = TRAIN ? A.hp + (int64_t)mem * 2 * A.bt * H : nullptr;
+  bf16* zp = TRAIN ? A.zp + (int64_t)mem * 2 * A.bt * H : nullptr;
+  // the first half of a layer's fragments, read before the barrier in front
+  // of its product
+  bf16x8 wt[8];
+  auto request = [&](const bf16x8* p) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) wt[k] = p[k * 64];
+  };
+  // 32 samples x 32 neurons: A from LDS rows, B the wave's fragments
+  auto product = [&](const bf16* act, const bf16x8* p) {
+    const bf16* a = act + (32 * m + (l & 31)) * LDA + 8 * h;
+    f32x16 acc = {};
+#pragma unroll
+    for (int k0 = 0; k0 < 16; k0 += 4) {
+      bf16x8 av[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) av[k] = *(const bf16x8*)(a + (k0 + k) * 16);
+      read_first();
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int kb = k0 + k;
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[k], wt[kb & 7], acc, 0, 0, 0);
+        if (kb < 8) wt[kb] = p[(kb + 8) * 64];
+      }
     }
-    if (!TB) {
-      const int kk = t >> 4, j = (t & 15) * 4;
-      for (int e = 0; e < 4; ++e) Bs[kk][j + e] = B[(int64_t)(k0 + kk) * ldb + n0 + j + e];
-    } else {
-      const int j = t >> 2, kk = (t & 3) * 4;
-      for (int e = 0; e < 4; ++e) Bs[kk + e][j] = B[(int64_t)(n0 + j) * ldb + k0 + kk + e];
-    }
-    __syncthreads();
-    bf16x8 a, b;
-    for (int j = 0; j < 8; ++j) {
-      a[j] = As[wm * 32 + (l & 31)][8 * (l >> 5) + j];
-      b[j] = Bs[8 * (l >> 5) + j][wn * 32 + (l & 31)];
-    }
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-    __syncthreads();
+    return acc;
+  };
+  request(tile(A.fw, 0));
+  if (t < 3 * H) {
+    ((float*)w4s)[t] = (float)wb[OFF_W4 + t];
+    w1s[t % 3][t / 3] = (float)wb[OFF_W1 + t];
+    bs[t >> 8][t & 255] = (float)wb[(t < H ? OFF_B1 : t < 2 * H ? OFF_B2 : OFF_B3) + (t & 255)];
+    if (t < 3) b4s[t] = (float)wb[OFF_B4 + t];
   }
-  for (int r = 0; r < 16; ++r) {
-    const int row = wm * 32 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
-    const int col = wn * 32 + (l & 31);
-    C[(int64_t)(m0 + row) * ldc + n0 + col] = acc[r];
+  if (t < TB) {
+    const int64_t j = A.order ? A.order[s0 + t] : s0 + t;
+    xs[t] = make_float4(A.X[3 * j], A.X[3 * j + 1], A.X[3 * j + 2], 0.0f);
+    if (TRAIN)
+      for (int k = 0; k < 3; ++k) ts[k][t] = A.T[3 * j + k];
   }
-}
-
-// layer 1: Z1 = W1 x + b1, H1 = act2(Z1) (bf16).  grid (Bt*256/256, 1, members)
-__global__ void k_in_fwd(int Bt, const float* X, const bf16* wb, float* Z1, bf16* H1,
-                         int64_t sZ) {
-  const int mem = blockIdx.z;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)Bt * H) return;
-  const int s = (int)(idx / H), n = (int)(idx % H);
-  const bf16* w = wb + (int64_t)mem * NPAD;
-  float z = (float)w[OFF_B1 + n];
-  for (int i = 0; i < 3; ++i) z += (float)w[OFF_W1 + n * 3 + i] * X[s * 3 + i];
-  Z1[mem * sZ + idx] = z;
-  H1[mem * sZ + idx] = (bf16)act2(z);
-}
-
-// Z += b (layer bias at boff), H = act2(Z), as bf16 (Hb) or fp32 (Hf)
-__global__ void k_bias_act(int Bt, const bf16* wb, int boff, float* Z, bf16* Hb, float* Hf,
-                           int64_t sZ) {
-  const int mem = blockIdx.z;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)Bt * H) return;
-  const int n = (int)(idx % H);
-  const float z = Z[mem * sZ + idx] + (float)wb[(int64_t)mem * NPAD + boff + n];
-  Z[mem * sZ + idx] = z;
-  if (Hb) Hb[mem * sZ + idx] = (bf16)act2(z);
-  if (Hf) Hf[mem * sZ + idx] = act2(z);
-}
-
-// output layer and loss: Y = W4 H3 + b4; dY = 2 (Y - T) / (3 Bt); loss sum
-__global__ void k_out_fwd(int Bt, const float* H3, const bf16* wb, const float* T, float* Y,
-                          float* dY, double* loss, int64_t sZ) {
-  const int mem = blockIdx.z;
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  double part = 0.0;
-  if (s < Bt) {
-    const bf16* w = wb + (int64_t)mem * NPAD;
-    const float* h = H3 + mem * sZ + (int64_t)s * H;
-    for (int k = 0; k < 3; ++k) {
-      float y = (float)w[OFF_B4 + k];
-      for (int n = 0; n < H; ++n) y += (float)w[OFF_W4 + k * H + n] * h[n];
-      const int64_t o = (int64_t)mem * Bt * 3 + s * 3 + k;
-      Y[o] = y;
-      if (T) {
-        const float d = y - T[s * 3 + k];
-        dY[o] = 2.0f * d / (3.0f * Bt);
-        part += (double)d * d;
+  lds_barrier();
+  // layer 1: thread t forms neuron t%256 of samples 16 (t/256) onward
+  bf16x8 v1[2];
+  {
+    const int n = t & 255, r0 = (t >> 8) * 16;
+    const float b = bs[0][n];
+    const float wi[3] = {w1s[0][n], w1s[1][n], w1s[2][n]};
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      bf16x8& v = v1[g];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int s = r0 + 8 * g + j;
+        const float4 x = xs[s];
+        float z = b;
+        z += wi[0] * x.x;
+        z += wi[1] * x.y;
+        z += wi[2] * x.z;
+        v[j] = (bf16)act2(z);
+        actA[s * LDA + n] = v[j];
       }
     }
   }
-  if (T && loss) {
-    for (int off = 32; off > 0; off >>= 1) part += __shfl_down(part, off);
-    if ((threadIdx.x & 63) == 0) atomicAdd(&loss[mem], part);
+  lds_barrier();
+  const int n = 32 * nt + (l & 31);  // this lane's neuron
+  // row of register r, and the fragment lane of four rows (q = r / 4)
+  auto row = [&](int r) { return 32 * m + 8 * (r >> 2) + 4 * h + (r & 3); };
+  auto frag4 = [&](bf16* base, int layer, int q) {
+    bf16x8* p = (bf16x8*)(base + (int64_t)layer * A.bt * H) +
+                ((int64_t)((s0 >> 4) + 2 * m + (q >> 1)) * 8 + nt) * 64 + (l & 31) + 32 * (q & 1);
+    return (bf16x4*)p + h;
+  };
+  // the four rows' fragments of an epilogue, until they are stored
+  bf16x4 held[4];
+  auto store_held = [&](bf16* base, int layer) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) *frag4(base, layer, q) = held[q];
+  };
+  f32x16 d2, d3;  // act2' of layers 2 and 3
+  // act2(z), and its derivative
+  auto act_d = [](float z, float& d) {
+    const float s = sig2(z);
+    d = s * (1.0f + LN2 * z * (1.0f - s));
+    return z * s;
+  };
+  // layer 2
+  {
+    const float b = bs[1][n];
+    const f32x16 acc = product(actA, tile(A.fw, 0));
+    if (TRAIN) {  // H1: eight samples of one neuron are one lane of a fragment
+      const int s = s0 + (t >> 8) * 16, n1 = t & 255;
+      bf16x8* f = (bf16x8*)hp + ((int64_t)(s >> 4) * 8 + (n1 >> 5)) * 64 + (n1 & 31);
+      f[0] = v1[0];
+      f[32] = v1[1];
+    }
+    request(tile(A.fw, 1));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      bf16x4& v = held[q];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int r = 4 * q + k;
+        float d;
+        v[k] = (bf16)act_d(acc[r] + b, d);
+        d2[r] = d;
+        actB[row(r) * LDA + n] = v[k];
+      }
+    }
+  }
+  lds_barrier();
+  // layer 3; its activation stays in FP32
+  {
+    const float b = bs[2][n];
+    const f32x16 acc = product(actB, tile(A.fw, 1));
+    if (TRAIN) store_held(hp, 1);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int r = 4 * q + k;
+        float d;
+        v[k] = act_d(acc[r] + b, d);
+        d3[r] = d;
+      }
+      *(float4*)&F[n * LDF + row(4 * q)] = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  }
+  lds_barrier();
+  // output layer: wave k < 3 forms output k of every sample, in neuron order
+  if (w < 3) {
+    float y = b4s[w];
+    // one dependent chain: 16 neurons are read while 16 are added, and the
+    // order is kept (left alone, each read is issued in front of its addition
+    // and waited for there: 12,000 cycles instead of 5,500)
+    float f0[8], f1[8];
+    float4 c0[2], c1[2];
+    auto read = [&](float* f, float4* c, int i) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) f[k] = F[(i + k) * LDF + l];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) c[k] = w4s[w][(i >> 2) + k];
+      read_first();
+    };
+    auto add = [&](const float* f, const float4* c) {
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        y += c[k].x * f[4 * k];
+        y += c[k].y * f[4 * k + 1];
+        y += c[k].z * f[4 * k + 2];
+        y += c[k].w * f[4 * k + 3];
+      }
+    };
+    read(f0, c0, 0);
+#pragma unroll 1
+    for (int i = 0; i < H; i += 16) {
+      read(f1, c1, i + 8);
+      add(f0, c0);
+      read(f0, c0, i + 16 < H ? i + 16 : 0);
+      add(f1, c1);
+    }
+    if (TRAIN) {
+      ds[w][l] = y - ts[w][l];
+    } else {
+      A.Y[((int64_t)mem * A.bt + s0 + l) * 3 + w] = y;
+    }
+  }
+  if (!TRAIN) return;
+  lds_barrier();
+  if (w == 0) {
+    double part = 0.0;
+    float g[3];
+    for (int k = 0; k < 3; ++k) {
+      const float d = ds[k][l];
+      g[k] = 2.0f * d / (3.0f * A.bt);
+      part += (double)d * d;
+    }
+    dys[l] = make_float4(g[0], g[1], g[2], 0.0f);
+    if (A.loss) {
+      for (int off = 32; off > 0; off >>= 1) part += __shfl_down(part, off);
+      if (l == 0) atomicAdd(&A.loss[mem], part);
+    }
+  }
+  lds_barrier();
+  float* part = A.part + ((int64_t)mem * (A.bt / TB) + chunk) * NSLOT_G * H;
+  // the sums over the 64 samples: 256 threads a sum, thread c neuron c
+  const int grp = t >> 8, c = t & 255;
+  // dZ3 = (dY W4) act2'(Z3)
+  request(tile(A.bw, 1));
+  {
+    const float* w4 = (const float*)w4s;
+    const float c0 = w4[n], c1 = w4[H + n], c2 = w4[2 * H + n];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      bf16x4& v = held[q];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int r = 4 * q + k;
+        const float4 dy = dys[row(r)];
+        const float g = dy.x * c0 + dy.y * c1 + dy.z * c2;
+        v[k] = (bf16)(g * d3[r]);
+        actA[row(r) * LDA + n] = v[k];
+      }
+    }
+  }
+  // shares of dW4 (a group an output) and db4
+  float share = 0.0f;
+  {
+    const float* dy = (const float*)dys;
+    float& v = share;
+    if (grp < 3) {
+#pragma unroll 1
+      for (int s = 0; s < TB; s += 8) {
+        float f[8], d[8];
+        *(float4*)f = *(const float4*)&F[c * LDF + s];
+        *(float4*)(f + 4) = *(const float4*)&F[c * LDF + s + 4];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) d[k] = dy[4 * (s + k) + grp];
+        read_first();
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v += d[k] * f[k];
+      }
+    } else if (c < 3) {
+      for (int s = 0; s < TB; ++s) v += dy[4 * s + c];
+    }
+  }
+  lds_barrier();
+  // dH2 = dZ3 W3, dZ2 = dH2 act2'(Z2); db3's shares
+  {
+    const f32x16 acc = product(actA, tile(A.bw, 1));
+    store_held(zp, 1);
+    if (grp < 3 || c < 3) part[(grp < 3 ? grp : 7) * H + c] = share;
+    request(tile(A.bw, 0));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      bf16x4& v = held[q];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int r = 4 * q + k;
+        v[k] = (bf16)(acc[r] * d2[r]);
+        actB[row(r) * LDA + n] = v[k];
+      }
+    }
+  }
+  if (grp == 0) {
+    float& b = share;
+    b = 0.0f;
+#pragma unroll 1
+    for (int s = 0; s < TB; s += 16) {
+      bf16 v[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) v[k] = actA[(s + k) * LDA + c];
+      read_first();
+#pragma unroll
+      for (int k = 0; k < 16; ++k) b += (float)v[k];
+    }
+  }
+  lds_barrier();
+  // dH1 = dZ2 W2, dZ1 = dH1 act2'(Z1) in FP32, Z1 formed again; db2's shares
+  {
+    const float b = bs[0][n];
+    const float wi[3] = {w1s[0][n], w1s[1][n], w1s[2][n]};
+    const f32x16 acc = product(actB, tile(A.bw, 0));
+    store_held(zp, 0);
+    if (grp == 0) part[8 * H + c] = share;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int r = 4 * q + k;
+        const float4 x = xs[row(r)];
+        float z = b;
+        z += wi[0] * x.x;
+        z += wi[1] * x.y;
+        z += wi[2] * x.z;
+        v[k] = acc[r] * dact2(z);
+      }
+      *(float4*)&F[n * LDF + row(4 * q)] = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  }
+  if (grp == 3) {
+    float b = 0.0f;
+#pragma unroll 1
+    for (int s = 0; s < TB; s += 16) {
+      bf16 v[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) v[k] = actB[(s + k) * LDA + c];
+      read_first();
+#pragma unroll
+      for (int k = 0; k < 16; ++k) b += (float)v[k];
+    }
+    part[9 * H + c] = b;
+  }
+  lds_barrier();
+  // shares of dW1 (a group an input) and db1
+  {
+    const float* x = (const float*)xs;
+    float v = 0.0f;
+#pragma unroll 1
+    for (int s = 0; s < TB; s += 8) {
+      float f[8], d[8];
+      *(float4*)f = *(const float4*)&F[c * LDF + s];
+      *(float4*)(f + 4) = *(const float4*)&F[c * LDF + s + 4];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) d[k] = x[4 * (s + k) + (grp < 3 ? grp : 0)];
+      read_first();
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v += grp < 3 ? f[k] * d[k] : f[k];
+    }
+    part[(3 + grp) * H + c] = v;
   }
 }
 
-// dH3 = dY W4, dZ3 = dH3 act2'(Z3) -> bf16
-__global__ void k_out_bwd(int Bt, const float* dY, const bf16* wb, const float* Z3, bf16* dZ3,
-                          int64_t sZ) {
-  const int mem = blockIdx.z;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)Bt * H) return;
-  const int s = (int)(idx / H), n = (int)(idx % H);
-  const bf16* w = wb + (int64_t)mem * NPAD;
-  const float* dy = dY + (int64_t)mem * Bt * 3 + s * 3;
-  const float g = dy[0] * (float)w[OFF_W4 + n] + dy[1] * (float)w[OFF_W4 + H + n] +
-                  dy[2] * (float)w[OFF_W4 + 2 * H + n];
-  dZ3[mem * sZ + idx] = (bf16)(g * dact2(Z3[mem * sZ + idx]));
+struct AdamArgs {
+  float *theta, *m1, *m2, *grad;  // [members][NPAD]
+  bf16 *wb, *fw, *bw;
+  float lr, b1, b2, eps, c1, c2;
+  int update;                     // 0: gradients alone
+};
+
+// Adam (Kingma & Ba 2015) on the FP32 master at o, whose value and moments are
+// given (read well before: a read after another element's store would wait for
+// memory at each element); the new value
+__device__ __forceinline__ float adam(const AdamArgs& P, int64_t o, float g, float th, float m1,
+                                      float m2) {
+  P.grad[o] = g;
+  const float a = P.b1 * m1 + (1.0f - P.b1) * g;
+  const float v = P.b2 * m2 + (1.0f - P.b2) * g * g;
+  P.m1[o] = a;
+  P.m2[o] = v;
+  const float p = th - P.lr * (a / P.c1) / (sqrtf(v / P.c2) + P.eps);
+  P.theta[o] = p;
+  P.wb[o] = (bf16)p;
+  return p;
 }
 
-// dZ = dH act2'(Z) -> bf16
-__global__ void k_act_bwd(int Bt, const float* dH, const float* Z, bf16* dZ, int64_t sZ) {
-  const int mem = blockIdx.z;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (int64_t)Bt * H) return;
-  dZ[mem * sZ + idx] = (bf16)(dH[mem * sZ + idx] * dact2(Z[mem * sZ + idx]));
+// where weight (out, in) of a layer sits in its fragments, forward and backward
+__host__ __device__ __forceinline__ int frag_fw(int out, int in) {
+  return (((out >> 5) * 16 + (in >> 4)) * 64 + (out & 31) + 32 * ((in >> 3) & 1)) * 8 + (in & 7);
+}
+__host__ __device__ __forceinline__ int frag_bw(int out, int in) {
+  return (((in >> 5) * 16 + (out >> 4)) * 64 + (in & 31) + 32 * ((out >> 3) & 1)) * 8 + (out & 7);
+}
+__global__ void k_weight_frags(const bf16* wb, bf16* fw, bf16* bw) {
+  const int mem = blockIdx.z, layer = blockIdx.y;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x, out = i >> 8, in = i & 255;
+  const bf16 v = wb[(int64_t)mem * NPAD + (layer ? OFF_W3 : OFF_W2) + i];
+  const int64_t o = ((int64_t)mem * 2 + layer) * PACKED;
+  fw[o + frag_fw(out, in)] = v;
+  bw[o + frag_bw(out, in)] = v;
 }
 
-// Batch reductions in two deterministic stages: per chunk of RCH samples
-// (grid x = chunk), then a sum over chunks in chunk order.
-constexpr int RCH = 64;
-constexpr int NPART = 8;  // partial slots per column
-
-// bias gradient partials: part[mem][c][n][slot] = sum over chunk of dZ[s][n]
-__global__ void k_colsum_part(int Bt, const bf16* dZ, float* part, int slot, int64_t sZ) {
-  const int mem = blockIdx.z, c = blockIdx.x, n = threadIdx.x;
-  const int chunks = Bt / RCH;
-  const bf16* p = dZ + mem * sZ + (int64_t)c * RCH * H;
-  float acc = 0.0f;
-  for (int s = 0; s < RCH; ++s) acc += (float)p[(int64_t)s * H + n];
-  part[(((int64_t)mem * chunks + c) * H + n) * NPART + slot] = acc;
-}
-
-// partials of dW4[k][n] = sum_s dY[s][k] H3[s][n] (slots 0..2), dW1[n][i] =
-// sum_s dZ1[s][n] X[s][i] (slots 3..5, dZ1 = dH1 act2'(Z1) in fp32), db1
-// (slot 6) and db4 (slot 7, columns 0..2)
-__global__ void k_small_part(int Bt, const float* dY, const float* H3, const float* dH1,
-                             const float* Z1, const float* X, float* part, int64_t sZ) {
-  const int mem = blockIdx.z, c = blockIdx.x, n = threadIdx.x;
-  const int chunks = Bt / RCH;
-  const float* h3 = H3 + mem * sZ;
-  const float* dh1 = dH1 + mem * sZ;
-  const float* z1 = Z1 + mem * sZ;
-  const float* dy = dY + (int64_t)mem * Bt * 3;
-  float w4[3] = {0, 0, 0}, w1[3] = {0, 0, 0}, b1 = 0.0f, b4 = 0.0f;
-  for (int s = c * RCH; s < (c + 1) * RCH; ++s) {
-    const float hv = h3[(int64_t)s * H + n];
-    for (int k = 0; k < 3; ++k) w4[k] += dy[s * 3 + k] * hv;
-    const float dz = dh1[(int64_t)s * H + n] * dact2(z1[(int64_t)s * H + n]);
-    b1 += dz;
-    for (int i = 0; i < 3; ++i) w1[i] += dz * X[s * 3 + i];
-    if (n < 3) b4 += dy[s * 3 + n];
+// Weight gradients dW[m][n] = sum_s dZ[s][m] H[s][n], one wave a 32 x 32 tile
+// with the whole batch in one MFMA chain (one wave's tile of one layer a CU for
+// two members: a wave reads 2 KB of fragments an MFMA, what a CU's path from
+// L2 carries in its 32 cycles), then Adam on the tile; further waves sum the
+// samples' shares of the small gradients.  Consecutive tiles go to one XCD, so
+// that an XCD's L2 reads two of the eight-odd megabytes and not all.
+// 4,096 samples, two members: 18 us, bound by the fragments' latency from L2
+// and beyond (24 of each operand in flight a wave; 8: 29 us); as a 64 x 64 GEMM
+// with both operands staged through LDS element by element 119 us a layer, and
+// 35 us for the sums.
+constexpr int WPF = 24;  // fragments of each operand in flight
+constexpr int SUMW = NSLOT_G * (H / 64);  // waves of a member's small sums
+__global__ __launch_bounds__(64) void k_train_weights(TrainArgs A, AdamArgs P) {
+  const int l = threadIdx.x, h = l >> 5;
+  const int tiles = 128 * A.members;  // 64 a layer and member
+  if ((int)blockIdx.x >= tiles) {
+    // small gradients: 64 samples' shares, in order
+    const int i = blockIdx.x - tiles, mem = i / SUMW, slot = (i % SUMW) >> 2,
+              n = 64 * (i & 3) + l;
+    const int chunks = A.bt / TB;
+    const float* q = A.part + ((int64_t)mem * chunks * NSLOT_G + slot) * H + n;
+    if (slot == 7 && n >= 3) return;
+    const int p = slot < 3   ? OFF_W4 + slot * H + n
+                  : slot < 6 ? OFF_W1 + n * 3 + slot - 3
+                             : (slot == 6   ? OFF_B1
+                                : slot == 7 ? OFF_B4
+                                : slot == 8 ? OFF_B3
+                                            : OFF_B2) + n;
+    const int64_t o = (int64_t)mem * NPAD + p;
+    const float th = P.theta[o], m1 = P.m1[o], m2 = P.m2[o];
+    float g = 0.0f;
+    for (int c0 = 0; c0 < chunks; c0 += 32) {
+      float v[32];
+#pragma unroll
+      for (int k = 0; k < 32; ++k)
+        v[k] = q[(int64_t)(c0 + k < chunks ? c0 + k : c0) * NSLOT_G * H];
+#pragma unroll
+      for (int k = 0; k < 32; ++k)
+        if (c0 + k < chunks) g += v[k];
+    }
+    if (P.update) adam(P, o, g, th, m1, m2);
+    else P.grad[o] = g;
+    return;
   }
-  float* q = part + (((int64_t)mem * chunks + c) * H + n) * NPART;
-  q[0] = w4[0]; q[1] = w4[1]; q[2] = w4[2];
-  q[3] = w1[0]; q[4] = w1[1]; q[5] = w1[2];
-  q[6] = b1;
-  q[7] = b4;
-}
-
-// second stages: sum the partials over chunks and scatter the gradients
-// (k_small_part's slots; k_colsum_part's slot 0 = b3, slot 1 = b2)
-__global__ void k_sum_small(int chunks, const float* part, float* grad) {
-  const int mem = blockIdx.z, n = threadIdx.x;
-  float v[NPART] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int c = 0; c < chunks; ++c) {
-    const float* q = part + (((int64_t)mem * chunks + c) * H + n) * NPART;
-    for (int k = 0; k < NPART; ++k) v[k] += q[k];
+  const int g = (blockIdx.x & 7) * (tiles >> 3) + (blockIdx.x >> 3);
+  const int mem = g >> 7, layer = (g >> 6) & 1, mt = (g >> 3) & 7, nt = g & 7;
+  const int KB = A.bt >> 4;
+  const int64_t lay = ((int64_t)mem * 2 + layer) * A.bt * H;
+  const bf16x8* za = (const bf16x8*)(A.zp + lay) + mt * 64 + l;
+  const bf16x8* hb = (const bf16x8*)(A.hp + lay) + nt * 64 + l;
+  // this lane's masters and moments (register r: row 8(r/4) + 4h + r%4)
+  const int in = 32 * nt + (l & 31);
+  const int64_t base = (int64_t)mem * NPAD + (layer ? OFF_W3 : OFF_W2);
+  float th[16], m1[16], m2[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int64_t o = base + (32 * mt + 8 * (r >> 2) + 4 * h + (r & 3)) * H + in;
+    th[r] = P.theta[o];
+    m1[r] = P.m1[o];
+    m2[r] = P.m2[o];
   }
-  float* g = grad + (int64_t)mem * NPAD;
-  for (int k = 0; k < 3; ++k) g[OFF_W4 + k * H + n] = v[k];
-  for (int i = 0; i < 3; ++i) g[OFF_W1 + n * 3 + i] = v[3 + i];
-  g[OFF_B1 + n] = v[6];
-  if (n < 3) g[OFF_B4 + n] = v[7];
-}
-
-__global__ void k_sum_bias(int chunks, const float* part, float* grad) {
-  const int mem = blockIdx.z, n = threadIdx.x;
-  float b3 = 0.0f, b2 = 0.0f;
-  for (int c = 0; c < chunks; ++c) {
-    const float* q = part + (((int64_t)mem * chunks + c) * H + n) * NPART;
-    b3 += q[0];
-    b2 += q[1];
+  f32x16 acc = {};
+  bf16x8 a[WPF], b[WPF];
+#pragma unroll
+  for (int i = 0; i < WPF; ++i)
+    if (i < KB) {
+      a[i] = za[i * 512];
+      b[i] = hb[i * 512];
+    }
+  for (int k0 = 0; k0 < KB; k0 += WPF) {
+#pragma unroll
+    for (int i = 0; i < WPF; ++i) {
+      if (k0 + i < KB) {
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], b[i], acc, 0, 0, 0);
+        if (k0 + i + WPF < KB) {
+          a[i] = za[(k0 + i + WPF) * 512];
+          b[i] = hb[(k0 + i + WPF) * 512];
+        }
+      }
+    }
   }
-  float* g = grad + (int64_t)mem * NPAD;
-  g[OFF_B3 + n] = b3;
-  g[OFF_B2 + n] = b2;
-}
-
-// Adam (Kingma & Ba 2015) on the FP32 masters; refreshes the BF16 copy
-__global__ void k_adam(float* theta, const float* grad, float* m1, float* m2, bf16* wb,
-                       float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int mem = blockIdx.z;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= NPARAM) return;
-  const int64_t o = (int64_t)mem * NPAD + i;
-  const float g = grad[o];
-  const float a = b1 * m1[o] + (1.0f - b1) * g;
-  const float v = b2 * m2[o] + (1.0f - b2) * g * g;
-  m1[o] = a;
-  m2[o] = v;
-  const float p = theta[o] - lr * (a / c1) / (sqrtf(v / c2) + eps);
-  theta[o] = p;
-  wb[o] = (bf16)p;
-}
-
-__global__ void k_gather(int bt, const int64_t* ord, const float* Xa, const float* Ta, float* Xb,
-                         float* Tb) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= bt) return;
-  const int64_t j = ord[i];
-  for (int k = 0; k < 3; ++k) {
-    Xb[3 * i + k] = Xa[3 * j + k];
-    Tb[3 * i + k] = Ta[3 * j + k];
+  const int64_t fo = ((int64_t)mem * 2 + layer) * PACKED;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    bf16x4 v;
+    const int out0 = 32 * mt + 8 * q + 4 * h;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int64_t o = base + (out0 + k) * H + in;
+      if (!P.update) {
+        P.grad[o] = acc[4 * q + k];
+        continue;
+      }
+      v[k] = (bf16)adam(P, o, acc[4 * q + k], th[4 * q + k], m1[4 * q + k], m2[4 * q + k]);
+      P.fw[fo + frag_fw(out0 + k, in)] = v[k];
+    }
+    if (P.update) *(bf16x4*)&P.bw[fo + frag_bw(out0, in)] = v;
   }
 }
 
@@ -401,69 +674,7 @@ __global__ void k_to_bf16(const float* theta, bf16* wb, int64_t n) {
   if (i < n) wb[i] = (bf16)theta[i];
 }
 
-// ---- fused inference -------------------------------------------------------------------
-// One kernel runs the whole ensemble forward pass, the disagreement test and
-// the baseline for a batch of queries; activations never leave registers.
-//
-// v_mfma_f32_32x32x16_bf16, 32 queries per wave: lane l holds query l%32 and
-// half h = l/32 of each activation.  A 32x32 output tile t leaves register r
-// of lane l holding neuron 32t + row32(r, h), row32(r, h) = 8(r/4) + 4h + r%4
-// (the D layout of the instruction: D[8(r/4)+4(l/32)+r%4][l%32]; A operand:
-// lane l holds row l%32, K indices 8(l/32)+j; B operand: column l%32, K
-// indices 8(l/32)+j).  Registers 8g..8g+7 of tile t form the B operand of
-// K-block kb = 2t+g of the next layer, so K index 8h + j of block kb is input
-// neuron pin32(kb, h, j) = 32(kb/2) + 16(kb%2) + 8(j/4) + 4h + j%4, and the
-// packed weights are P[t][kb][lane][j] = W[32t + lane%32][pin32(kb, lane/32,
-// j)].  A block of IW waves stages one member's packed 256x256 layer (128
-// KB) in LDS and its waves (IW x 32 queries) read the A fragments from
-// there, so L2 supplies each weight once per block instead of once per wave;
-// each fragment read from LDS feeds a 32-query MFMA.
-constexpr int MAXM = 4;   // largest ensemble
-
-struct InferArgs {
-  int64_t n;
-  int members;
-  const bf16* wb;         // [members][NPAD]
-  const bf16* packed;     // [members][2][PACKED]: layers 2 and 3
-  const bf16* p1;         // [members][16*64*8]: layer-1 A operands
-  const float* norm;      // shift[3], scale[3]
-  float thresh;           // relative member deviation that sends a query to the fallback
-  const float* prep;      // [n][8] k_prep's features and baselines
-  float* out;             // [n][3] physical outputs (T_b, |omega_d|, latitude)
-  float* raw;             // optional [members][n][3] normalised outputs
-  int32_t* flag;          // [n] in: k_prep's side | near << 1; out: 1 = fallback
-};
-
-// one member's small parameters, staged in LDS: b1, b2, b3, w4 (one float4
-// of the three output weights per layer-3 neuron), b4
-struct SmallW {
-  float b1[H], b2[H], b3[H];
-  float4 w4[H];
-  float b4[4];
-};
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-// the biases of one 32x32 output tile in a lane's accumulator order: register
-// r holds neuron row32(r, h), so b points at the tile's bias + 4h and the 16
-// values are four float4 runs at 8-element strides
-__device__ __forceinline__ f32x16 bias16(const float* b) {
-  f32x16 acc;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const float4 v = *(const float4*)(b + 8 * q);
-    acc[4 * q] = v.x;
-    acc[4 * q + 1] = v.y;
-    acc[4 * q + 2] = v.z;
-    acc[4 * q + 3] = v.w;
-  }
-  return acc;
-}
-
-__device__ __forceinline__ int pin32(int kb, int h, int j) {
-  return 32 * (kb >> 1) + 16 * (kb & 1) + 8 * (j >> 2) + 4 * h + (j & 3);
-}
-__device__ __forceinline__ int row32(int r, int h) { return 8 * (r >> 2) + 4 * h + (r & 3); }
-
+// ---- inference: packing and pre-pass (the kernel: rapt_mlp_infer.hip) ---------------------
 __global__ void k_pack(const bf16* wb, bf16* packed, int woff) {
   const int mem = blockIdx.z;
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
@@ -478,7 +689,6 @@ __global__ void k_pack(const bf16* wb, bf16* packed, int woff) {
 // hi_j and 3 <= j < 6 multiplies W1[.][j-3] by lo_{j-3}: the product with the
 // bf16 weights is as accurate as the FP32 vector form.  A operand of tile t
 // (32 neurons), lane (h, j): W1[32t + l%32][j%3] for h = 0, j < 6, else 0.
-constexpr int P1SIZE = 8 * 64 * 8;  // bf16 elements of one member's layer-1 operands
 __global__ void k_pack1(const bf16* wb, bf16* p1) {
   const int mem = blockIdx.z;
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;  // 8 tiles * 64 lanes * 8
@@ -510,203 +720,6 @@ __global__ void k_prep(int64_t n, const float* query, SplitC S, double mass, dou
   float4* o = (float4*)(prep + 8 * i);
   o[0] = make_float4(x[0], x[1], x[2], b.lnT);
   o[1] = make_float4(b.lnW, b.lnLat, 0.0f, 0.0f);
-}
-
-// IW = 8 waves per block (two per SIMD), 32 queries per wave.  The biases
-// start the accumulators.  Staging is pipelined: each member's two 256x256
-// layers pass through LDS as four 64 KB halves (layer 2 tiles 0-3, 4-7, then
-// layer 3), alternating between two buffers; while the waves compute with
-// one half, the next half (the next member's, or member 0's for the next
-// chunk) streams into the other buffer with direct global-to-LDS loads, so
-// the loads never wait on a barrier with the matrix cores idle.  A half is
-// 64 fragments of 1 KB; wave w loads fragments 8i + w.
-constexpr int IW = 8;
-constexpr int QW = 32;  // queries per wave
-constexpr int HALF = PACKED / 16;  // bf16x8 elements of half a packed layer (64 KB)
-
-// stage s of a member's four: layer 2 + (s >> 1), fragments 64 (s & 1) onward.
-// Wave wv loads fragments 8i + wv, starting at i = rot (the block's rotation,
-// so that the CUs of an XCD do not all ask the L2 for the same lines at the
-// same moment).  The loads go through a buffer resource
-// (buffer_load_dwordx4 ... lds), which counts on vmcnt alone: with the FLAT
-// form (global_load_lds) in flight the compiler must treat the LDS counter as
-// unordered, and every LDS read of the half being computed would then wait
-// for all reads issued before it.
-__device__ __forceinline__ void stage_load(__amdgpu_buffer_rsrc_t rs, int m, int s, bf16x8* buf,
-                                           int wv, int l, int rot) {
-  const int base = (m * 2 + (s >> 1)) * PACKED * 2 + (s & 1) * HALF * 16;  // bytes
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int f = 8 * ((i + rot) & 7) + wv;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-        rs, (__attribute__((address_space(3))) void*)(buf + 64 * f), 16,
-        base + (64 * f + l) * 16, 0, 0, 0);
-  }
-}
-
-__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0); }
-
-// one 32x32 output tile of a hidden layer from the fragments of buf (tile
-// t of the half: fragments 16 t .. 16 t + 15).  The A fragments are read
-// PF ahead into a ring of registers, so each MFMA's LDS read has PF - 1
-// matrix operations of cover (the compiler's own schedule gives one).
-constexpr int PF = 4;
-__device__ __forceinline__ f32x16 tile32(const bf16x8* buf, int t, const bf16x8* in,
-                                         f32x16 acc, int l) {
-  const bf16x8* p = buf + 16 * t * 64 + l;
-  bf16x8 a[PF];
-#pragma unroll
-  for (int i = 0; i < PF; ++i) a[i] = p[i * 64];
-#pragma unroll
-  for (int kb = 0; kb < 16; ++kb) {
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kb % PF], in[kb], acc, 0, 0, 0);
-    if (kb + PF < 16) a[kb % PF] = p[(kb + PF) * 64];
-  }
-  // keep that order in the schedule (left alone, the scheduler sinks each
-  // read next to its MFMA to save registers): PF LDS reads (mask 0x100),
-  // then per step one MFMA (0x008), one LDS read and up to five other
-  // vector instructions (0x002)
-  __builtin_amdgcn_sched_group_barrier(0x100, PF, 0);
-#pragma unroll
-  for (int kb = 0; kb < 16; ++kb) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-    if (kb + PF < 16) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
-  }
-  return acc;
-}
-
-__global__ __launch_bounds__(IW * 64) void k_infer(InferArgs A) {
-  __shared__ bf16x8 buf0[HALF], buf1[HALF];
-  __shared__ SmallW sw[MAXM];
-  const int l = threadIdx.x & 63, wv = threadIdx.x >> 6, h = l >> 5;
-  const int64_t groups = (A.n + QW - 1) / QW;
-  const int64_t chunks = (groups + IW - 1) / IW;
-  if ((int64_t)blockIdx.x >= chunks) return;  // no work: no barrier is reached
-  for (int m = 0; m < A.members; ++m) {
-    const bf16* w = A.wb + (int64_t)m * NPAD;
-    for (int i = threadIdx.x; i < H; i += IW * 64) {
-      sw[m].b1[i] = (float)w[OFF_B1 + i];
-      sw[m].b2[i] = (float)w[OFF_B2 + i];
-      sw[m].b3[i] = (float)w[OFF_B3 + i];
-      sw[m].w4[i] = make_float4((float)w[OFF_W4 + i], (float)w[OFF_W4 + H + i],
-                                (float)w[OFF_W4 + 2 * H + i], 0.0f);
-    }
-    if (threadIdx.x < 3) sw[m].b4[threadIdx.x] = (float)w[OFF_B4 + threadIdx.x];
-  }
-  // the packed layers 2 and 3 of every member as a raw buffer (stride 0,
-  // the gfx9 word-3 format bits); reads past the end return 0
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)A.packed, (short)0, A.members * 2 * PACKED * (int)sizeof(bf16), 0x00020000);
-  const int rot = blockIdx.x & 7;
-  stage_load(rs, 0, 0, buf0, wv, l, rot);
-  for (int64_t ch = blockIdx.x; ch < chunks; ch += gridDim.x) {
-    const int64_t g = ch * IW + wv;
-    const int64_t qi = g * QW + (l & 31);
-    const bool valid = g < groups && qi < A.n;
-    const float4* pq = (const float4*)(A.prep + 8 * (valid ? qi : 0));
-    const float4 p0 = pq[0];
-    const float xin[3] = {p0.x, p0.y, p0.z};
-    const int rg = valid ? A.flag[qi] : 0;  // k_prep's side | near << 1
-    bf16x8 xb;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) xb[j] = (bf16)0.0f;
-    if (h == 0) {
-#pragma unroll
-      for (int j = 0; j < 3; ++j) {
-        const bf16 hv = (bf16)xin[j];
-        xb[j] = hv;
-        xb[3 + j] = (bf16)(xin[j] - (float)hv);
-      }
-    }
-    float mean[3] = {0.0f, 0.0f, 0.0f}, lo[3], hi[3];
-    for (int c = 0; c < 3; ++c) { lo[c] = 3.0e38f; hi[c] = -3.0e38f; }
-    for (int m = 0; m < A.members; ++m) {
-      const SmallW& W = sw[m];
-      const bf16x8* P1 = (const bf16x8*)(A.p1 + (int64_t)m * P1SIZE);
-      const int mn = m + 1 < A.members ? m + 1 : 0;  // the member whose layer 2 comes next
-      // layer 1 (its operands come from global memory)
-      bf16x8 act[16];
-      wait_loads();
-      __syncthreads();  // first pass: sw written; every pass: this member's half 0 landed
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        f32x16 acc = bias16(&W.b1[32 * t + 4 * h]);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(P1[t * 64 + l], xb, acc, 0, 0, 0);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) act[2 * t + (r >> 3)][r & 7] = (bf16)act2(acc[r]);
-      }
-      // layer 2, tiles 0-3 from buf0 while tiles 4-7 stream into buf1
-      stage_load(rs, m, 1, buf1, wv, l, rot);
-      bf16x8 nxt[16];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        f32x16 acc = tile32(buf0, t, act, bias16(&W.b2[32 * t + 4 * h]), l);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) nxt[2 * t + (r >> 3)][r & 7] = (bf16)act2(acc[r]);
-      }
-      wait_loads();
-      __syncthreads();  // buf1 landed; buf0 free
-      stage_load(rs, m, 2, buf0, wv, l, rot);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        f32x16 acc = tile32(buf1, t, act, bias16(&W.b2[32 * (t + 4) + 4 * h]), l);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) nxt[2 * (t + 4) + (r >> 3)][r & 7] = (bf16)act2(acc[r]);
-      }
-      wait_loads();
-      __syncthreads();  // layer 3 half 0 in buf0; buf1 free
-      stage_load(rs, m, 3, buf1, wv, l, rot);
-      // layer 3 and the output layer (FP32)
-      float o0 = 0.0f, o1 = 0.0f, o2 = 0.0f;
-#pragma unroll
-      for (int half = 0; half < 2; ++half) {
-        if (half == 1) {
-          wait_loads();
-          __syncthreads();  // layer 3 half 1 in buf1; buf0 free
-          stage_load(rs, mn, 0, buf0, wv, l, rot);
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int tt = 4 * half + t;
-          f32x16 acc = tile32(half ? buf1 : buf0, t, nxt, bias16(&W.b3[32 * tt + 4 * h]), l);
-#pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const float4 c = W.w4[32 * tt + row32(r, h)];
-            const float v = act2(acc[r]);
-            // fused multiply-adds (the library compiles without contraction)
-            o0 = __builtin_fmaf(c.x, v, o0);
-            o1 = __builtin_fmaf(c.y, v, o1);
-            o2 = __builtin_fmaf(c.z, v, o2);
-          }
-        }
-      }
-      o0 += __shfl_xor(o0, 32);
-      o1 += __shfl_xor(o1, 32);
-      o2 += __shfl_xor(o2, 32);
-      const float o[3] = {o0 + W.b4[0], o1 + W.b4[1], o2 + W.b4[2]};
-      for (int c = 0; c < 3; ++c) {
-        mean[c] += o[c];
-        lo[c] = fminf(lo[c], o[c]);
-        hi[c] = fmaxf(hi[c], o[c]);
-      }
-      if (A.raw && valid && l < 32)
-        for (int c = 0; c < 3; ++c) A.raw[((int64_t)m * A.n + qi) * 3 + c] = o[c];
-    }
-    if (valid && l < 32) {
-      const float4 p1 = pq[1];
-      const float bb[3] = {p0.w, p1.x, p1.y};
-      int bad = (rg & 2) ? 1 : 0;
-      for (int k = 0; k < 3; ++k) {
-        const float sc = A.norm[3 + k];
-        const float mu = mean[k] / (float)A.members;
-        if (expm1f(sc * fmaxf(hi[k] - mu, mu - lo[k])) > A.thresh) bad = 1;
-        A.out[qi * 3 + k] = expf(bb[k] + A.norm[k] + sc * mu);
-      }
-      A.flag[qi] = bad;
-    }
-  }
-  wait_loads();  // the prefetch issued for a chunk this block does not run
 }
 
 // targets: normalised log-residuals from traced labels (T_b, omega_d, lat)
@@ -751,22 +764,18 @@ struct rapt_mlp {
   float* norm = nullptr;
   bool packed_ok = false;
   SplitC split{};  // regime of the drift label (rapt_mlp_set_split)
-  // training workspace (batch-sized)
-  float *X = nullptr, *T = nullptr, *Z1 = nullptr, *Z2 = nullptr, *Z3 = nullptr;
-  float *H3 = nullptr, *dH = nullptr, *Y = nullptr, *dY = nullptr;
-  bf16 *H1 = nullptr, *H2 = nullptr, *dZb = nullptr;
-  float *partS = nullptr, *partB = nullptr;
+  // training: weight fragments (k_train_rows), and the batch-sized workspace
+  bf16 *fw = nullptr, *bw = nullptr;
+  bf16 *hp = nullptr, *zp = nullptr;
+  float *part = nullptr, *X = nullptr, *Y = nullptr;
   double* loss = nullptr;
 };
 
 static void mlp_free_work(rapt_mlp* m) {
-  void* p[] = {m->X, m->T, m->Z1, m->Z2, m->Z3, m->H3, m->dH, m->Y, m->dY,
-               m->H1, m->H2, m->dZb, m->partS, m->partB, m->loss};
+  void* p[] = {m->hp, m->zp, m->part, m->X, m->Y};
   for (void* q : p) (void)hipFree(q);
-  m->X = m->T = m->Z1 = m->Z2 = m->Z3 = m->H3 = m->dH = m->Y = m->dY = nullptr;
-  m->partS = m->partB = nullptr;
-  m->H1 = m->H2 = m->dZb = nullptr;
-  m->loss = nullptr;
+  m->hp = m->zp = nullptr;
+  m->part = m->X = m->Y = nullptr;
   m->batch = 0;
 }
 
@@ -774,22 +783,13 @@ static int mlp_work(rapt_mlp* m, int bt) {
   if (m->batch == bt) return RAPT_OK;
   mlp_free_work(m);
   rapt_ctx* c = m->ctx;
-  const size_t act = (size_t)m->members * bt * H;
+  const size_t act = (size_t)m->members * 2 * bt * H;
   bool ok = hipMalloc(&m->X, sizeof(float) * 3 * bt) == hipSuccess &&
-            hipMalloc(&m->T, sizeof(float) * 3 * bt) == hipSuccess &&
-            hipMalloc(&m->Z1, sizeof(float) * act) == hipSuccess &&
-            hipMalloc(&m->Z2, sizeof(float) * act) == hipSuccess &&
-            hipMalloc(&m->Z3, sizeof(float) * act) == hipSuccess &&
-            hipMalloc(&m->H3, sizeof(float) * act) == hipSuccess &&
-            hipMalloc(&m->dH, sizeof(float) * act) == hipSuccess &&
             hipMalloc(&m->Y, sizeof(float) * 3 * bt * m->members) == hipSuccess &&
-            hipMalloc(&m->dY, sizeof(float) * 3 * bt * m->members) == hipSuccess &&
-            hipMalloc(&m->H1, sizeof(bf16) * act) == hipSuccess &&
-            hipMalloc(&m->H2, sizeof(bf16) * act) == hipSuccess &&
-            hipMalloc(&m->dZb, sizeof(bf16) * act) == hipSuccess &&
-            hipMalloc(&m->partS, sizeof(float) * (act / RCH) * NPART) == hipSuccess &&
-            hipMalloc(&m->partB, sizeof(float) * (act / RCH) * NPART) == hipSuccess &&
-            hipMalloc(&m->loss, sizeof(double) * m->members) == hipSuccess;
+            hipMalloc(&m->hp, sizeof(bf16) * act) == hipSuccess &&
+            hipMalloc(&m->zp, sizeof(bf16) * act) == hipSuccess &&
+            hipMalloc(&m->part, sizeof(float) * m->members * (bt / TB) * NSLOT_G * H) ==
+                hipSuccess;
   if (!ok) {
     mlp_free_work(m);
     return set_err(c, RAPT_E_OOM, "MLP workspace allocation failed");
@@ -798,56 +798,19 @@ static int mlp_work(rapt_mlp* m, int bt) {
   return RAPT_OK;
 }
 
-// forward of a training batch already in m->X; T may be null (no loss)
-static void mlp_forward(rapt_mlp* m, int bt, bool with_loss) {
-  hipStream_t st = m->ctx->stream;
-  const int mem = m->members;
-  const int64_t sZ = (int64_t)bt * H;
-  const dim3 ew((unsigned)((sZ + 255) / 256), 1, mem);
-  const dim3 gg(H / 64, bt / 64, mem);
-  hipLaunchKernelGGL(k_in_fwd, ew, dim3(256), 0, st, bt, m->X, m->wb, m->Z1, m->H1, sZ);
-  // Z2 = H1 W2^T
-  hipLaunchKernelGGL((k_gemm<false, true>), gg, dim3(256), 0, st, bt, H, H, m->H1, H, sZ,
-                     m->wb + OFF_W2, H, (int64_t)NPAD, m->Z2, H, sZ);
-  hipLaunchKernelGGL(k_bias_act, ew, dim3(256), 0, st, bt, m->wb, OFF_B2, m->Z2, m->H2,
-                     (float*)nullptr, sZ);
-  hipLaunchKernelGGL((k_gemm<false, true>), gg, dim3(256), 0, st, bt, H, H, m->H2, H, sZ,
-                     m->wb + OFF_W3, H, (int64_t)NPAD, m->Z3, H, sZ);
-  hipLaunchKernelGGL(k_bias_act, ew, dim3(256), 0, st, bt, m->wb, OFF_B3, m->Z3,
-                     (bf16*)nullptr, m->H3, sZ);
-  hipLaunchKernelGGL(k_out_fwd, dim3((unsigned)((bt + 255) / 256), 1, mem), dim3(256), 0, st,
-                     bt, m->H3, m->wb, with_loss ? m->T : (const float*)nullptr, m->Y, m->dY,
-                     m->loss, sZ);
-}
-
-static void mlp_backward(rapt_mlp* m, int bt) {
-  hipStream_t st = m->ctx->stream;
-  const int mem = m->members;
-  const int64_t sZ = (int64_t)bt * H;
-  const int chunks = bt / RCH;
-  const dim3 ew((unsigned)((sZ + 255) / 256), 1, mem);
-  const dim3 gw(H / 64, H / 64, mem);   // 256 x 256 weight gradients
-  const dim3 ga(H / 64, bt / 64, mem);  // batch x 256 activation gradients
-  const dim3 gr(chunks, 1, mem);        // per-chunk partial reductions
-  // layer 3
-  hipLaunchKernelGGL(k_out_bwd, ew, dim3(256), 0, st, bt, m->dY, m->wb, m->Z3, m->dZb, sZ);
-  hipLaunchKernelGGL((k_gemm<true, false>), gw, dim3(256), 0, st, H, H, bt, m->dZb, H, sZ,
-                     m->H2, H, sZ, m->grad + OFF_W3, H, (int64_t)NPAD);
-  hipLaunchKernelGGL(k_colsum_part, gr, dim3(256), 0, st, bt, m->dZb, m->partB, 0, sZ);
-  hipLaunchKernelGGL((k_gemm<false, false>), ga, dim3(256), 0, st, bt, H, H, m->dZb, H, sZ,
-                     m->wb + OFF_W3, H, (int64_t)NPAD, m->dH, H, sZ);
-  // layer 2
-  hipLaunchKernelGGL(k_act_bwd, ew, dim3(256), 0, st, bt, m->dH, m->Z2, m->dZb, sZ);
-  hipLaunchKernelGGL((k_gemm<true, false>), gw, dim3(256), 0, st, H, H, bt, m->dZb, H, sZ,
-                     m->H1, H, sZ, m->grad + OFF_W2, H, (int64_t)NPAD);
-  hipLaunchKernelGGL(k_colsum_part, gr, dim3(256), 0, st, bt, m->dZb, m->partB, 1, sZ);
-  hipLaunchKernelGGL(k_sum_bias, dim3(1, 1, mem), dim3(256), 0, st, chunks, m->partB, m->grad);
-  hipLaunchKernelGGL((k_gemm<false, false>), ga, dim3(256), 0, st, bt, H, H, m->dZb, H, sZ,
-                     m->wb + OFF_W2, H, (int64_t)NPAD, m->dH, H, sZ);
-  // layer 1 and the output layer
-  hipLaunchKernelGGL(k_small_part, gr, dim3(256), 0, st, bt, m->dY, m->H3, m->dH, m->Z1, m->X,
-                     m->partS, sZ);
-  hipLaunchKernelGGL(k_sum_small, dim3(1, 1, mem), dim3(256), 0, st, chunks, m->partS, m->grad);
+static TrainArgs train_args(const rapt_mlp* m, int bt) {
+  TrainArgs A;
+  memset(&A, 0, sizeof A);
+  A.bt = bt;
+  A.members = m->members;
+  A.wb = m->wb;
+  A.fw = m->fw;
+  A.bw = m->bw;
+  A.hp = m->hp;
+  A.zp = m->zp;
+  A.part = m->part;
+  A.Y = m->Y;
+  return A;
 }
 
 extern "C" {
@@ -871,6 +834,9 @@ int rapt_mlp_create(rapt_ctx* c, int32_t members, const float* theta0, double ma
             hipMalloc(&m->wb, sizeof(bf16) * np) == hipSuccess &&
             hipMalloc(&m->packed, sizeof(bf16) * members * 2 * PACKED) == hipSuccess &&
             hipMalloc(&m->p1, sizeof(bf16) * members * P1SIZE) == hipSuccess &&
+            hipMalloc(&m->fw, sizeof(bf16) * members * 2 * PACKED) == hipSuccess &&
+            hipMalloc(&m->bw, sizeof(bf16) * members * 2 * PACKED) == hipSuccess &&
+            hipMalloc(&m->loss, sizeof(double) * members) == hipSuccess &&
             hipMalloc(&m->norm, sizeof(float) * 6) == hipSuccess;
   if (!ok) {
     rapt_mlp_destroy(m);
@@ -887,6 +853,8 @@ int rapt_mlp_create(rapt_ctx* c, int32_t members, const float* theta0, double ma
     }
   hipLaunchKernelGGL(k_to_bf16, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, st, m->theta,
                      m->wb, (int64_t)np);
+  hipLaunchKernelGGL(k_weight_frags, dim3(H * H / 256, 2, members), dim3(256), 0, st, m->wb,
+                     m->fw, m->bw);
   hipLaunchKernelGGL(k_zero_f, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, st, m->m1,
                      (int64_t)np);
   hipLaunchKernelGGL(k_zero_f, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, st, m->m2,
@@ -906,7 +874,8 @@ int rapt_mlp_destroy(rapt_mlp* m) {
   if (!m) return RAPT_E_ARG;
   if (m->ctx) (void)hipSetDevice(m->ctx->device);
   mlp_free_work(m);
-  void* p[] = {m->theta, m->grad, m->m1, m->m2, m->wb, m->packed, m->p1, m->norm};
+  void* p[] = {m->theta, m->grad, m->m1, m->m2, m->wb, m->packed, m->p1, m->norm,
+               m->fw, m->bw, m->loss};
   for (void* q : p) (void)hipFree(q);
   delete m;
   return RAPT_OK;
@@ -993,53 +962,55 @@ int rapt_mlp_train(rapt_mlp* m, int64_t n, const float* X, const float* T, int32
   int rc = mlp_work(m, batch);
   if (rc) return rc;
   hipStream_t st = c->stream;
-  float *dXall = nullptr, *dTall = nullptr;
-  int64_t* dorder = nullptr;
   const int64_t nidx = (int64_t)steps * batch;
-  if (hipMalloc(&dXall, sizeof(float) * 3 * n) != hipSuccess ||
-      hipMalloc(&dTall, sizeof(float) * 3 * n) != hipSuccess ||
-      hipMalloc(&dorder, sizeof(int64_t) * (nidx > 0 ? nidx : 1)) != hipSuccess) {
-    (void)hipFree(dXall);
-    (void)hipFree(dTall);
-    (void)hipFree(dorder);
-    return set_err(c, RAPT_E_OOM, "training data allocation failed");
-  }
   for (int64_t i = 0; i < nidx; ++i)
-    if (order[i] < 0 || order[i] >= n) {
-      (void)hipFree(dXall);
-      (void)hipFree(dTall);
-      (void)hipFree(dorder);
+    if (order[i] < 0 || order[i] >= n)
       return set_err(c, RAPT_E_ARG, "sample index out of range");
-    }
+  Workspace ws(c);
+  char* mem = ws.get(sizeof(int64_t) * nidx + sizeof(float) * 6 * n);
+  if (!mem) return set_err(c, RAPT_E_OOM, "training data allocation failed");
+  int64_t* dorder = (int64_t*)mem;
+  float *dX = (float*)(dorder + nidx), *dT = dX + 3 * n;
   rc = RAPT_OK;
-  if (hipMemcpyAsync(dXall, X, sizeof(float) * 3 * n, hipMemcpyHostToDevice, st) != hipSuccess ||
-      hipMemcpyAsync(dTall, T, sizeof(float) * 3 * n, hipMemcpyHostToDevice, st) != hipSuccess ||
+  if (hipMemcpyAsync(dX, X, sizeof(float) * 3 * n, hipMemcpyHostToDevice, st) != hipSuccess ||
+      hipMemcpyAsync(dT, T, sizeof(float) * 3 * n, hipMemcpyHostToDevice, st) != hipSuccess ||
       (nidx > 0 && hipMemcpyAsync(dorder, order, sizeof(int64_t) * nidx, hipMemcpyHostToDevice,
                                   st) != hipSuccess))
     rc = set_err(c, RAPT_E_HIP, "training data copy failed");
-  const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+  AdamArgs P;
+  memset(&P, 0, sizeof P);
+  P.theta = m->theta;
+  P.m1 = m->m1;
+  P.m2 = m->m2;
+  P.grad = m->grad;
+  P.wb = m->wb;
+  P.fw = m->fw;
+  P.bw = m->bw;
+  P.b1 = 0.9f;
+  P.b2 = 0.999f;
+  P.eps = 1e-8f;
+  P.update = lr0 > 0.0f ? 1 : 0;
+  TrainArgs A = train_args(m, batch);
+  A.X = dX;
+  A.T = dT;
   for (int s = 0; s < steps && rc == RAPT_OK; ++s) {
-    // gather the batch
-    hipLaunchKernelGGL(k_gather, dim3((batch + 255) / 256), dim3(256), 0, st, batch,
-                       dorder + (int64_t)s * batch, dXall, dTall, m->X, m->T);
     const bool last = s == steps - 1;
-    if (last && loss_out)
-      hipLaunchKernelGGL(k_zero_d, dim3(1), dim3(64), 0, st, m->loss, m->members);
-    mlp_forward(m, batch, true);
-    mlp_backward(m, batch);
+    A.order = dorder + (int64_t)s * batch;
+    A.loss = last && loss_out ? m->loss : nullptr;
+    if (A.loss) hipLaunchKernelGGL(k_zero_d, dim3(1), dim3(64), 0, st, m->loss, m->members);
+    // cosine learning-rate schedule from lr0 to lr1 over this call
+    const float frac = steps > 1 ? (float)s / (float)(steps - 1) : 0.0f;
+    P.lr = lr1 + 0.5f * (lr0 - lr1) * (1.0f + cosf(3.14159265f * frac));
+    ++m->step;
+    P.c1 = 1.0f - powf(P.b1, (float)m->step);
+    P.c2 = 1.0f - powf(P.b2, (float)m->step);
+    hipLaunchKernelGGL(k_train_rows<true>, dim3(batch / TB, 1, m->members), dim3(RT), 0, st, A);
+    hipLaunchKernelGGL(k_train_weights, dim3((128 + SUMW) * m->members), dim3(64), 0, st, A, P);
     if (last && grad_out)
       for (int k = 0; k < m->members; ++k)
         if (hipMemcpyAsync(grad_out + (size_t)k * NPARAM, m->grad + (size_t)k * NPAD,
                            sizeof(float) * NPARAM, hipMemcpyDeviceToHost, st) != hipSuccess)
           rc = set_err(c, RAPT_E_HIP, "gradient copy failed");
-    // cosine learning-rate schedule from lr0 to lr1 over this call
-    const float frac = steps > 1 ? (float)s / (float)(steps - 1) : 0.0f;
-    const float lr = lr1 + 0.5f * (lr0 - lr1) * (1.0f + cosf(3.14159265f * frac));
-    ++m->step;
-    const float c1 = 1.0f - powf(b1, (float)m->step), c2 = 1.0f - powf(b2, (float)m->step);
-    if (lr0 > 0.0f)
-      hipLaunchKernelGGL(k_adam, dim3((NPARAM + 255) / 256, 1, m->members), dim3(256), 0, st,
-                         m->theta, m->grad, m->m1, m->m2, m->wb, lr, b1, b2, eps, c1, c2);
   }
   if (rc == RAPT_OK && loss_out) {
     double lh[16];
@@ -1051,9 +1022,6 @@ int rapt_mlp_train(rapt_mlp* m, int64_t n, const float* X, const float* T, int32
   if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
     rc = rc ? rc : set_err(c, RAPT_E_HIP, "training kernels failed");
   m->packed_ok = false;
-  (void)hipFree(dXall);
-  (void)hipFree(dTall);
-  (void)hipFree(dorder);
   return rc;
 }
 
@@ -1068,8 +1036,7 @@ int rapt_mlp_get_params(rapt_mlp* m, float* theta) {
   return RAPT_OK;
 }
 
-// Forward pass through the training path (GEMM kernels) for n <= workspace
-// batch rows of features X; Y out [members][n][3].
+// Forward pass through the training path for n <= workspace batch rows of features X; Y out [members][n][3].
 int rapt_mlp_forward(rapt_mlp* m, int64_t n, const float* X, float* Y) {
   if (!m || n <= 0 || !X || !Y) return m ? set_err(m->ctx, RAPT_E_ARG, "bad forward call")
                                          : RAPT_E_ARG;
@@ -1082,7 +1049,9 @@ int rapt_mlp_forward(rapt_mlp* m, int64_t n, const float* X, float* Y) {
   hipLaunchKernelGGL(k_zero_f, dim3((unsigned)((3 * bt + 255) / 256)), dim3(256), 0, st, m->X,
                      (int64_t)3 * bt);
   HIP_OK(c, hipMemcpyAsync(m->X, X, sizeof(float) * 3 * n, hipMemcpyHostToDevice, st));
-  mlp_forward(m, bt, false);
+  TrainArgs A = train_args(m, bt);
+  A.X = m->X;
+  hipLaunchKernelGGL(k_train_rows<false>, dim3(bt / TB, 1, m->members), dim3(RT), 0, st, A);
   HIP_OK(c, hipGetLastError());
   for (int k = 0; k < m->members; ++k)
     HIP_OK(c, hipMemcpyAsync(Y + (size_t)k * n * 3, m->Y + (size_t)k * bt * 3,
@@ -1139,14 +1108,10 @@ int rapt_mlp_infer(rapt_mlp* m, int64_t n, const float* query, float thresh, flo
     A.flag = dflag;
     int dev_cus = 256;
     (void)hipDeviceGetAttribute(&dev_cus, hipDeviceAttributeMultiprocessorCount, c->device);
-    // persistent: one block per CU, each taking chunks of IW x QW queries
-    const int64_t groups = (n + QW - 1) / QW;
-    int64_t blocks = (groups + IW - 1) / IW;
-    if (blocks > dev_cus) blocks = dev_cus;
     HIP_OK(c, hipEventRecord(c->ev0, st));
     hipLaunchKernelGGL(k_prep, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, dq,
                        m->split, m->mass, m->eV, dprep, dflag);
-    hipLaunchKernelGGL(k_infer, dim3((unsigned)blocks), dim3(IW * 64), 0, st, A);
+    rapt_launch_infer(st, A, dev_cus);
     HIP_OK(c, hipEventRecord(c->ev1, st));
     if (hipGetLastError() != hipSuccess ||
         hipMemcpyAsync(out, dout, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, st) !=
