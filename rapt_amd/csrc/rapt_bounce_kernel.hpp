@@ -111,15 +111,6 @@ struct LineRHS {
   }
 };
 
-// a / b given r = rcp_nr(b): the compiler's division sequence without the
-// scaling of extreme exponents, so the same (correctly rounded) quotient for
-// the magnitudes of field lines; several quotients share a denominator.
-__device__ __forceinline__ double div_r(double a, double b, double r) {
-  const double q = a * r;
-  return __builtin_fma(__builtin_fma(-b, q, a), r, q);
-}
-__device__ __forceinline__ double div_nr(double a, double b) { return div_r(a, b, rcp_nr(b)); }
-
 // de Boor's BSPLVB for k = 2: the three splines that are not 0 at s in
 // [ka, kb), whose neighbouring knots are kz <= ka and kb <= kc
 struct Basis {

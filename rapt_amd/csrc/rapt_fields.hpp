@@ -116,6 +116,16 @@ __device__ __forceinline__ double rcp_nr(double x) {
   e = __builtin_fma(-x, r, 1.0);
   return __builtin_fma(r, e, r);
 }
+// a / b given r = rcp_nr(b): the compiler's division sequence without its
+// scaling of extreme exponents, so the same (correctly rounded) quotient where
+// it and the reciprocal are normal numbers, in 4 operations (9 with the
+// reciprocal) instead of 12; several quotients share a denominator.
+// v_div_fixup_f64 gives zeros, infinities and NaNs the division's own results.
+__device__ __forceinline__ double div_r(double a, double b, double r) {
+  const double q = a * r;
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), r, q), b, a);
+}
+__device__ __forceinline__ double div_nr(double a, double b) { return div_r(a, b, rcp_nr(b)); }
 // single precision: v_rsq_f32 / v_rcp_f32 are accurate to about 1 ulp
 __device__ __forceinline__ float rsqrt_nr(float x) { return __builtin_amdgcn_rsqf(x); }
 __device__ __forceinline__ float rcp_nr(float x) { return __builtin_amdgcn_rcpf(x); }
@@ -609,12 +619,13 @@ __device__ __forceinline__ double timescale(const FieldC& F, double t, double x,
 // ---- right-hand sides ---------------------------------------------------------
 // Lorentz force, the eom closure of Particle.advance (rapt/Particle.py:284-298).
 // gm is gamma*m: frozen at advance start for static fields, else recomputed.
-template <int M>
+// SP: a static field and no equatorial constraint, compiled in.
+template <int M, bool SP = false>
 __device__ __forceinline__ void rhs_lorentz(const FieldC& F, double charge, double mass,
                                             double& gm, bool eq, double t, const double* Y,
                                             double* out) {
   const V3 p{Y[3], Y[4], Y[5]};
-  if (!F.is_static) gm = __builtin_sqrt(mass * mass + dot3(p, p) / C_LIGHT_SQ);
+  if (!SP && !F.is_static) gm = __builtin_sqrt(mass * mass + dot3(p, p) / C_LIGHT_SQ);
   const double ig = rcp_nr(gm);
   out[0] = p.x * ig;
   out[1] = p.y * ig;
@@ -631,7 +642,7 @@ __device__ __forceinline__ void rhs_lorentz(const FieldC& F, double charge, doub
     out[4] = charge * (c.y * ig);
     out[5] = charge * (c.z * ig);
   }
-  if (eq) {
+  if (!SP && eq) {
     out[2] = 0.0;
     out[5] = 0.0;
   }

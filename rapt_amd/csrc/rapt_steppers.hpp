@@ -15,6 +15,8 @@
 #include <hip/hip_runtime.h>
 #endif
 
+#include "rapt_fields.hpp"
+
 namespace rapt {
 
 constexpr double UROUND = 2.3e-16;
@@ -306,7 +308,7 @@ __device__ __forceinline__ double dop853_attempt(RHS& f, double x, double h, con
                            b11, k2[i], b12, k3[i]);
     y1[i] = __builtin_fma(h, bs, y[i]);
     const double sk = atol + rtol * fmax(err_mag<N, G>(y, i), err_mag<N, G>(y1, i));
-    const double isk = 1.0 / sk;
+    const double isk = div_nr(1.0, sk);
     const double e3 = fsum_acc(bs, -bhh1, k1[i], -bhh2, k9[i], -bhh3, k3[i]) * isk;
     err2 = __builtin_fma(e3, e3, err2);
     const double e5 = fsum(er1, k1[i], er6, k6[i], er7, k7[i], er8, k8[i], er9, k9[i],
@@ -315,7 +317,7 @@ __device__ __forceinline__ double dop853_attempt(RHS& f, double x, double h, con
   }
   double deno = err + 0.01 * err2;
   if (deno <= 0.0) deno = 1.0;
-  return __builtin_fabs(h) * err * __builtin_sqrt(1.0 / (N * deno));
+  return __builtin_fabs(h) * err * __builtin_sqrt(div_nr(1.0, N * deno));
 }
 
 // ---- HINIT (initial step guess) ----------------------------------------------

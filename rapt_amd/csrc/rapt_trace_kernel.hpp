@@ -38,7 +38,8 @@ namespace rapt {
 
 // ---- right-hand-side functors --------------------------------------------------
 // P = RAPT_PREC_FP64 or RAPT_PREC_FP32_FIELD (field and drift terms in float)
-template <int M, int P>
+// SP: a static field without the equatorial constraint, compiled in
+template <int M, int P, bool SP>
 struct LorentzRHS {
   const FieldC& F;
   double charge, mass, gm;
@@ -48,7 +49,7 @@ struct LorentzRHS {
     if constexpr (P == RAPT_PREC_FP32_FIELD) {
       rhs_lorentz_f32<M>(F, charge, mass, gm, eq, t, y, o);
     } else {
-      rhs_lorentz<M>(F, charge, mass, gm, eq, t, y, o);
+      rhs_lorentz<M, SP>(F, charge, mass, gm, eq, t, y, o);
     }
     ++nf;
   }
@@ -76,9 +77,13 @@ struct GcRHS {
 };
 
 // ---- the persistent tracer kernel ---------------------------------------------------
-// SP: for KIND_GC, the instantiation for the Tao-Chan-Brizard equations in a
-// static field (those choices compiled in); the generic one reads A.eom and
-// F.is_static.
+// SP (trace_use_sp): the instantiation for a static field, with the
+// Tao-Chan-Brizard equations (KIND_GC and KIND_ADAPTIVE) and without the
+// equatorial constraint (KIND_PARTICLE and KIND_ADAPTIVE): those choices
+// compiled in, where the generic one reads A.eom, A.eq and F.is_static.  A
+// Lorentz right-hand side that decides at run time forms gamma m (a division
+// and a square root, 32 instructions of ~95) and its reciprocal in every stage
+// and throws them away in a static field.
 // Register budget: two waves per SIMD (256 registers per lane) for the
 // analytic fields, where it costs 12-92 bytes of spills per lane in the GC
 // and Particle kernels and hides the dependent-chain latency better (one-lane
@@ -256,7 +261,7 @@ void k_trace(KArgs A) {
     // ---- f0 = f(x, y) at a call start without a carried FSAL stage ------------
     if (active && !k1ok) {
       if (!gcmode) {
-        LorentzRHS<M, P> f{F, charge, mass, gm, A.eq != 0, 0};
+        LorentzRHS<M, P, SP> f{F, charge, mass, gm, A.eq != 0, 0};
         if (stepper != RAPT_STEP_RKF45) f(x, y, k1);
         gm = f.gm;
         c_fcn += f.nf;
@@ -270,7 +275,7 @@ void k_trace(KArgs A) {
     // ---- HINIT on the first call of an advance (first_step == 0) -------------
     if (active && h == 0.0) {
       if (!gcmode) {
-        LorentzRHS<M, P> f{F, charge, mass, gm, A.eq != 0, 0};
+        LorentzRHS<M, P, SP> f{F, charge, mass, gm, A.eq != 0, 0};
         h = hinit<6, P == RAPT_PREC_FP32_FIELD>(f, x, y, k1, stepper == RAPT_STEP_DOP853 ? 8 : 5, hmax, A.atol, A.rtol);
         gm = f.gm;
         c_fcn += f.nf;
@@ -304,12 +309,14 @@ void k_trace(KArgs A) {
       }
     }
     // ---- one full step attempt --------------------------------------------------
-    double y1[6], k7[6], err = 0.0, fob = 1.0;
+    double y1[6], k7[6], err = 0.0, fob = 1.0, rfob = 1.0;
     if (stepping) {
-      if (stepper != RAPT_STEP_RKF45)
+      if (stepper != RAPT_STEP_RKF45) {
         fob = ctl_fob(((stepper == RAPT_STEP_DOP853) ? A.c853 : A.c5).beta, lfo);
+        rfob = rcp_nr(fob);
+      }
       if (!gcmode) {
-        LorentzRHS<M, P> f{F, charge, mass, gm, A.eq != 0, 0};
+        LorentzRHS<M, P, SP> f{F, charge, mass, gm, A.eq != 0, 0};
         if (KIND == KIND_ADAPTIVE || stepper == RAPT_STEP_DOP853) {
           err = dop853_attempt<6, P == RAPT_PREC_FP32_FIELD>(f, x, h, y, k1, y1, A.atol, A.rtol);
         } else {
@@ -331,7 +338,7 @@ void k_trace(KArgs A) {
     }
     // DOP853: the 12th evaluation f(x+h, y1) only after acceptance
     if (KIND != KIND_GC && stepping && !gcmode && stepper == RAPT_STEP_DOP853 && err <= 1.0) {
-      LorentzRHS<M, P> f{F, charge, mass, gm, A.eq != 0, 0};
+      LorentzRHS<M, P, SP> f{F, charge, mass, gm, A.eq != 0, 0};
       f(x + h, y1, k7);
       gm = f.gm;
       c_fcn += f.nf;
@@ -366,9 +373,10 @@ void k_trace(KArgs A) {
         const CtlParams& C = (stepper == RAPT_STEP_DOP853) ? A.c853 : A.c5;
         const double l2e = log2(err);
         const double fac11 = exp2(C.expo1 * l2e);
-        double fac = fac11 / fob;
-        fac = fmax(C.facc2, fmin(C.facc1, fac / C.safe));
-        double hnew = h / fac;
+        const double rsafe = rcp_nr(C.safe);
+        double fac = div_r(fac11, fob, rfob);
+        fac = fmax(C.facc2, fmin(C.facc1, div_r(fac, C.safe, rsafe)));
+        double hnew = div_nr(h, fac);
         if (err <= 1.0) {
           lfo = fmax(l2e, LFO0);
           ++nacc_call;
@@ -390,7 +398,7 @@ void k_trace(KArgs A) {
             h = hnew;
           }
         } else {
-          hnew = h / fmin(C.facc1, fac11 / C.safe);
+          hnew = div_nr(h, fmin(C.facc1, div_r(fac11, C.safe, rsafe)));
           reject = true;
           if (nacc_call >= 1) ++c_rej;
           last = false;
@@ -563,11 +571,11 @@ __global__ __launch_bounds__(256) void k_rhs_eval(FieldC F, int mode, int eom, i
   }
 }
 
-// the one-lane GC kernel's TCB + static-field instantiation applies
-// (VarEarthDipole is never static)
+// the SP instantiation of a run's kind applies (VarEarthDipole is never static)
 template <int M>
 static inline bool trace_use_sp(const KArgs& A) {
-  return M != F_VAR_EARTH_DIPOLE && A.eom == EOM_TCB && A.F.is_static != 0;
+  return M != F_VAR_EARTH_DIPOLE && A.F.is_static != 0 &&
+         (A.kind == KIND_PARTICLE || A.eom == EOM_TCB) && (A.kind == KIND_GC || A.eq == 0);
 }
 
 }  // namespace rapt

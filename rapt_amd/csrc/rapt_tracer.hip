@@ -192,7 +192,8 @@ __global__ void k_fill_u64(unsigned long long* p, int n) {
 template <int M, int K>
 static void launch_trace(rapt_ctx* c, const KArgs& A, int block, int64_t lanes) {
   const int64_t g = (lanes + block - 1) / block;
-  if constexpr (K == KIND_GC && M != F_VAR_EARTH_DIPOLE) {
+  // (an interpreted user-written field's time is the interpreter's)
+  if constexpr (M != F_VAR_EARTH_DIPOLE && (K == KIND_GC || M != F_EXPR)) {
     if (trace_use_sp<M>(A)) {
       hipLaunchKernelGGL((k_trace<M, K, RAPT_PREC_FP64, true>), dim3((unsigned)g), dim3(block),
                          0, c->stream, A);
