@@ -581,12 +581,13 @@ __device__ __forceinline__ void gcn_body(const KArgs& A, const int qown) {
     }
     Y4 y1{}, k7{};
     double err = 0.0;
-    double fob = 1.0;
+    double fob = 1.0, rfob = 1.0;
     if (stepping) {
       fob = ctl_fob(C.beta, lfo);
+      rfob = rcp_nr(fob);
       using namespace dp5;
       Y4 k2{}, k3{}, k4{}, k5{}, k6{};
-#pragma unroll 1
+#pragma unroll
       for (int s = 2; s <= 7; ++s) {
         Y4 ts;
         double xs;
@@ -634,7 +635,7 @@ __device__ __forceinline__ void gcn_body(const KArgs& A, const int qown) {
         const double e = (e1 * k1.c[i] + e3 * k3.c[i] + e4 * k4.c[i] + e5 * k5.c[i] +
                           e6 * k6.c[i] + e7 * k7.c[i]) * h;
         const double sk = A.atol + A.rtol * fmax(__builtin_fabs(y.c[i]), __builtin_fabs(y1.c[i]));
-        es.c[i] = e / sk;
+        es.c[i] = div_nr(e, sk);
       }
       err = __builtin_sqrt(grp_sumsq<L>(es) * (1.0 / 4));
     }
@@ -643,9 +644,10 @@ __device__ __forceinline__ void gcn_body(const KArgs& A, const int qown) {
       if (q == 0) ++c_stp;
       const double l2e = log2(err);
       const double fac11 = exp2(C.expo1 * l2e);
-      double fac = fac11 / fob;
-      fac = fmax(C.facc2, fmin(C.facc1, fac / C.safe));
-      double hnew = h / fac;
+      const double rsafe = rcp_nr(C.safe);
+      double fac = div_r(fac11, fob, rfob);
+      fac = fmax(C.facc2, fmin(C.facc1, div_r(fac, C.safe, rsafe)));
+      double hnew = div_nr(h, fac);
       if (err <= 1.0) {
         lfo = fmax(l2e, LFO0);
         ++nacc_call;
@@ -664,7 +666,7 @@ __device__ __forceinline__ void gcn_body(const KArgs& A, const int qown) {
           h = hnew;
         }
       } else {
-        hnew = h / fmin(C.facc1, fac11 / C.safe);
+        hnew = div_nr(h, fmin(C.facc1, div_r(fac11, C.safe, rsafe)));
         reject = true;
         if (nacc_call >= 1 && q == 0) ++c_rej;
         last = false;
