@@ -552,8 +552,9 @@ __device__ __forceinline__ int32_t line_pair(const BounceArgs& A, const QuadTab&
         }
         const double val = 1.0 - div_r(sp(s), Bm, rBm);
         const double w = tw[e0 + k];
-        ts[k] = w / __builtin_sqrt(val);
-        ti[k] = want_eye ? w * __builtin_sqrt(fmax(val, 0.0)) : 0.0;
+        const double sq = __builtin_sqrt(val);
+        ts[k] = div_nr(w, sq);
+        ti[k] = val > 0.0 ? w * sq : 0.0;
       }
       if (g == 0) {
 #pragma unroll
