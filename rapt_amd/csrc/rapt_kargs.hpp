@@ -27,7 +27,8 @@ struct CtlParams {  // scipy set_integrator knobs of one stepper
 struct KArgs {
   FieldC F;
   int32_t kind, eom, stepper, nmax;
-  int32_t eq, check, width, pad;
+  int32_t eq, check, width;
+  int32_t wave_lanes;  // KIND_ADAPTIVE: lanes of each wave that take particles
   double rtol, atol, gc_rtol, gc_atol;
   CtlParams c853, c5;
   double max_step, first_step;

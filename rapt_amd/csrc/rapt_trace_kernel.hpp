@@ -102,7 +102,8 @@ void k_trace(KArgs A) {
   const int eom = SP ? (int)EOM_TCB : A.eom;
   const FieldC& F = A.F;
   const int64_t n = cold()->n;
-  bool active = false, exhausted = false;
+  bool active = false,
+       exhausted = KIND == KIND_ADAPTIVE && (int)(threadIdx.x & 63) >= cold()->wave_lanes;
   int64_t pi = 0;
   // per-lane particle + integrator state
   double x = 0, y[6] = {0, 0, 0, 0, 0, 0}, k1[6] = {0, 0, 0, 0, 0, 0};

@@ -736,6 +736,23 @@ int rapt_batch_set_rows(rapt_batch* b, int32_t width, const int64_t* row_cap) {
 
 }  // extern "C"
 
+// Lanes of a wave that take particles in an ADAPTIVE run: as few as leave
+// `waves` waves for the launch, a power of two.  A wave's step runs every path
+// that any of its particles takes, here a full-orbit step, a guiding-centre step,
+// an adiabaticity test and a conversion, so a launch that does not fill the GPU
+// is faster with its particles spread over more waves, up to one a SIMD
+// (current-sheet protons, spread so and packed: 100 3.7 and 7.9 ms, 500 4.3 and
+// 9.1, 4,096 7.5 and 9.6, 32,768 8.7 and 9.3; with two waves a SIMD 4,096 take
+// 8.1 and 32,768 11.3).
+// Full-orbit and guiding-centre runs take one path and are not: 4,096 protons
+// 6.3 ms packed and 7.6 spread, 1,000 guiding centres on octets 5.0 and 6.3.
+static constexpr int SPREAD_WAVES = 4;  // waves a CU: one a SIMD
+static int spread_lanes(int64_t n, int64_t waves) {
+  int wl = 64;
+  while (wl > 1 && (n + wl / 2 - 1) / (wl / 2) <= waves) wl /= 2;
+  return wl;
+}
+
 // lanes_per_particle 0 of a guiding-centre run: octets, whose step is the
 // shortest, while they leave a SIMD one wave (advance(4) of DoubleDipole
 // electrons, octets and quads: 16 3.3 and 3.8 ms, 1,000 5.0 and 5.9, 8,192 5.5
@@ -871,7 +888,14 @@ static int prepare_run(rapt_batch* b, const rapt_trace_desc* d, KArgs& A, int& b
   // at 65,536 (four waves per CU) the two are equal for the analytic dipole
   // and 64 was slower on a gridded one.  The grouped kernels count the lanes
   // of all their groups.
+  int cus = 0;
+  HIP_OK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
   int block = d->block > 0 ? d->block : 0;
+  A.wave_lanes = 64;
+  if (d->mode == RAPT_MODE_ADAPTIVE && d->lanes <= 0) {
+    A.wave_lanes = spread_lanes(b->n, (int64_t)SPREAD_WAVES * cus);
+    lanes = (b->n + A.wave_lanes - 1) / A.wave_lanes * 64;
+  }
   if (block == 0) {
     int64_t launched = lanes;
     if (grouped) {
@@ -885,8 +909,6 @@ static int prepare_run(rapt_batch* b, const rapt_trace_desc* d, KArgs& A, int& b
         launched = (groups < b->n ? groups : b->n) * L;
       }
     }
-    int cus = 0;
-    HIP_OK(c, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device));
     block = launched < (int64_t)4 * 64 * cus ? 64 : 256;
   }
   block_out = block;
