@@ -103,13 +103,15 @@ typedef struct {
     double delta;                /* advance(delta) */
     int64_t lanes;               /* resident lanes of the persistent grid (0 = auto);
                                     fewer lanes than particles turns on work refill */
-    int32_t lanes_per_particle;  /* GC with DOPRI5 in FP64: 4 (default, 0) spreads one
-                                    guiding centre over a lane quad, 2 over a lane pair,
-                                    8 over a lane octet; 1 = one lane per particle;
+    int32_t lanes_per_particle;  /* GC with DOPRI5 in FP64: 4 spreads one guiding centre
+                                    over a lane quad, 2 over a lane pair, 8 over a lane
+                                    octet; 1 = one lane per particle;
                                     3 = mixed: the first mixed_quads particles of the
                                     work order on lane quads, the rest on lane pairs;
                                     5 = mixed: the first mixed_octets on octets, the
-                                    next mixed_quads on quads, the rest on pairs.
+                                    next mixed_quads on quads, the rest on pairs;
+                                    0 (default) = by the number of particles, with the
+                                    resident lanes (quads where lanes is given).
                                     Results do not depend on it */
     int32_t work_order;          /* 0: the batch's queue order (shortest output step
                                     first, or by cost after rapt_batch_set_cost); 1:

@@ -753,12 +753,54 @@ static int spread_lanes(int64_t n, int64_t waves) {
   return wl;
 }
 
-// lanes_per_particle 0 of a guiding-centre run: octets, whose step is the
-// shortest, while they leave a SIMD one wave (advance(4) of DoubleDipole
-// electrons, octets and quads: 16 3.3 and 3.8 ms, 1,000 5.0 and 5.9, 8,192 5.5
-// and 6.3; 32,768 8.5 and 8.3), else quads.
-static int default_group(const rapt_ctx* c, int64_t n) {
-  return n <= 8192 && c->field.model != RAPT_FIELD_EXPR ? 8 : 4;
+// The layout of a guiding-centre run with lanes_per_particle 0 and lanes 0.  A
+// lone wave issues an instruction in nearly every slot of its SIMD, so what
+// counts is the instructions of a particle's step (pairs 92, quads 116, octets
+// 200), a step's length for the longest particles (shortest on octets), and
+// that the longest particles' waves share their SIMD with no other: one wave a
+// SIMD, each lane group taking particles from the queue, ends sooner than two
+// that slow each other down and have nothing to refill from.  `one` lanes are a
+// wave a SIMD (65,536).  DoubleDipole electrons, advance(10), output step 1 s,
+// quads all resident as before, then this layout, ms:
+//   octets, one wave a SIMD, up to `one` / 4:  10,000 14.5, 12.4; 16,384 14.7, 12.9
+//   quads, one wave a SIMD, up to `one` / 2:   24,576 17.0, 15.1; 32,768 18.4, 15.2
+//   pairs and, for the costliest, quads (as many as fit beside the pairs' chains:
+//   fewer the more particles there are), one wave a SIMD, up to 3/2 `one`:
+//                       40,000 19.3, 15.2; 65,536 22.4, 18.4; 98,304 29.1, 26.3
+//   pairs, two waves a SIMD (each has particles enough to even out):
+//            131,072 36.4, 31.4; 262,144 69.7, 55.8; 524,288 136, 105
+// and the same way in the dipole, and with output steps of a bounce period.  In
+// input order the front of the queue is not the costliest, and a gridded field
+// waits for memory, which a second wave hides: quads there (65,536: 21.8 against
+// 22.6, and 45 against 83 on a grid), octets for few (8,192 10.0, 8.2; a grid's
+// 16,384 29.9, 23.1).
+static void default_layout(const rapt_ctx* c, rapt_trace_desc& d, int64_t n, bool ordered) {
+  if (d.mode != RAPT_MODE_GC || d.stepper != RAPT_STEP_DOPRI5 ||
+      d.precision != RAPT_PREC_FP64 || d.lanes_per_particle != 0 || d.lanes > 0 ||
+      d.mixed_quads < 0 || c->field.model == RAPT_FIELD_EXPR)
+    return;
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess)
+    return;
+  const int64_t one = (int64_t)256 * cus;
+  const bool grid = c->field.model == RAPT_FIELD_GRID;
+  ordered = ordered && d.work_order == 0;
+  if (n <= (ordered ? one / 4 : one / 8)) {
+    d.lanes_per_particle = 8;
+    d.lanes = one;
+  } else if (!ordered || grid) {
+    d.lanes_per_particle = 4;
+    return;
+  } else if (n <= one / 2) {
+    d.lanes_per_particle = 4;
+    d.lanes = one;
+  } else {
+    const int64_t quads = (3 * one / 2 - n) / 8;
+    d.lanes_per_particle = 3;
+    d.mixed_quads = quads > 0 ? quads : 1;
+    d.lanes = quads > 0 ? one : 2 * one;
+  }
+  if (d.block == 0) d.block = 64;
 }
 
 // Validates a descriptor and builds the kernel arguments of a batch run.
@@ -982,7 +1024,7 @@ int rapt_batch_run(rapt_batch* b, const rapt_trace_desc* desc, rapt_counters* cn
   rapt_ctx* c = b->ctx;
   rapt_trace_desc dd = *desc;
   const rapt_trace_desc* d = &dd;
-  if (dd.lanes_per_particle == 0) dd.lanes_per_particle = default_group(c, b->n);
+  default_layout(c, dd, b->n, true);
   KArgs A;
   int block = 256;
   int64_t lanes = 0;
@@ -1074,7 +1116,7 @@ int rapt_trace_device_noalloc(rapt_ctx* c, const rapt_trace_desc* d, int64_t n,
   // a user-written field: one lane per particle (compiled if an earlier run
   // loaded that kernel, else interpreted; loading a module allocates)
   if (c->field.model == RAPT_FIELD_EXPR) dd.lanes_per_particle = 1;
-  if (dd.lanes_per_particle == 0) dd.lanes_per_particle = default_group(c, n);
+  default_layout(c, dd, n, order != nullptr);
   KArgs A;
   int block = 256;
   int64_t lanes = 0;
@@ -1156,7 +1198,7 @@ int rapt_batch_epochs_begin(rapt_batch* b, const rapt_trace_desc* desc,
   rapt_ctx* c = b->ctx;
   rapt_trace_desc dd = *desc;
   const rapt_trace_desc* d = &dd;
-  if (dd.lanes_per_particle == 0) dd.lanes_per_particle = default_group(c, b->n);
+  default_layout(c, dd, b->n, true);
   if (rows_per_epoch < 1) return set_err(c, RAPT_E_ARG, "rows_per_epoch must be >= 1");
   const int width = d->mode == RAPT_MODE_PARTICLE ? 7 : (d->mode == RAPT_MODE_GC ? 5 : 8);
   rapt_batch_epochs_end(b);

@@ -61,11 +61,12 @@ def test_adaptive_particles_spread_over_waves(n):
           batch.advance_adaptive(*arg, params=prm, lanes=n + 63 & ~63))
 
 
-@pytest.mark.parametrize("n", [1, 9, 8192, 8193])
+@pytest.mark.parametrize("n", [1, 9, 8193, 16385, 32769, 98305])
 def test_default_guiding_centre_layout_and_order(n):
-    """Octets up to 8,192, quads above, taken in the order of r / v where the
-    output steps are equal; against one lane a particle in input order (one
-    step differs by a part in 1e12 from the rest) and other rows left alone."""
+    """Octets up to 16,384, quads up to 32,768, quads and pairs up to 98,304 and
+    pairs above, taken in the order of r / v where the output steps are equal;
+    against one lane a particle, and that in input order (one step differs by a
+    part in 1e12 from the rest)."""
     w = W.doubledipole_electrons_gc(n=n)
     f = F.DoubleDipole()
     v = w["v"]
