@@ -389,6 +389,10 @@ int rapt_mlp_forward(rapt_mlp *m, int64_t n, const float *X, float *Y);
  * raw [members][n][3] optional; kernel_ms: inference kernel time. */
 int rapt_mlp_infer(rapt_mlp *m, int64_t n, const float *query, float thresh, float *out,
                    int32_t *flag, float *raw, double *kernel_ms);
+/* the same with the values in double precision, the second (the drift's
+ * angular velocity) times sign */
+int rapt_mlp_infer_values(rapt_mlp *m, int64_t n, const float *query, float thresh, double sign,
+                          double *out, int32_t *flag, float *raw, double *kernel_ms);
 
 /* ---- device-resident batch (replaces one scipy ode loop per particle) -- */
 int rapt_batch_create(rapt_ctx *ctx, int64_t n, rapt_batch **out);

@@ -110,6 +110,8 @@ def lib():
     L.rapt_mlp_get_params.argtypes = [vp, fp]
     L.rapt_mlp_forward.argtypes = [vp, C.c_int64, fp, fp]
     L.rapt_mlp_infer.argtypes = [vp, C.c_int64, fp, C.c_float, fp, i32p, fp, dp]
+    L.rapt_mlp_infer_values.argtypes = [vp, C.c_int64, fp, C.c_float, C.c_double, dp, i32p, fp,
+                                        dp]
     L.rapt_batch_create.argtypes = [vp, C.c_int64, C.POINTER(vp)]
     L.rapt_batch_destroy.argtypes = [vp]
     L.rapt_batch_upload.argtypes = [vp, dp, i32p]
@@ -139,7 +141,7 @@ def lib():
                "rapt_batch_epochs_begin", "rapt_batch_epoch_next", "rapt_batch_epochs_end",
                "rapt_mlp_create", "rapt_mlp_destroy",
                "rapt_mlp_set_norm", "rapt_mlp_set_split", "rapt_mlp_targets", "rapt_mlp_train", "rapt_mlp_get_params",
-               "rapt_mlp_forward", "rapt_mlp_infer",
+               "rapt_mlp_forward", "rapt_mlp_infer", "rapt_mlp_infer_values",
                "rapt_batch_create", "rapt_batch_destroy", "rapt_batch_upload",
                "rapt_batch_set_rows", "rapt_batch_run", "rapt_batch_download", "rapt_trace",
                "rapt_batch_reset", "rapt_batch_set_cost", "rapt_eye", "rapt_particle_gc",

@@ -48,7 +48,7 @@ def _run(field, mode, state, flags, row_cap, desc, device=0, max_launches=64, gr
     ctx.set_field(field.descriptor())
     n = state.shape[1]
     width = N.ROW_WIDTH[mode]
-    rows = [[] for _ in range(n)]
+    rows = [np.zeros((0, width))] * n
     idx = np.arange(n)
     cur_state, cur_flags, cur_cap = state.copy(), flags.copy(), np.asarray(row_cap, np.int64)
     final_state = state.copy()
@@ -70,11 +70,13 @@ def _run(field, mode, state, flags, row_cap, desc, device=0, max_launches=64, gr
         for k in ("naccpt", "nrejct", "nstep", "nfcn", "nswitch"):
             tot[k] += getattr(cnt, k)
         tot["kernel_ms"] += cnt.kernel_ms
-        off = b.row_off
-        for j, i in enumerate(idx):
-            m = out["nrows"][j]
-            if m:
-                rows[i].append(out["rows"][off[j]:off[j] + m])
+        buf = out["rows"]
+        ends = zip(idx.tolist(), b.row_off.tolist(), out["nrows"].tolist())
+        if launches == 1:
+            rows = [buf[o:o + m].copy() for _, o, m in ends]
+        else:
+            for i, o, m in ends:
+                rows[i] = np.concatenate([rows[i], buf[o:o + m]])
         final_state[:, idx] = out["state"]
         final_flags[idx] = out["flags"]
         status[idx] = out["status"]
@@ -88,7 +90,6 @@ def _run(field, mode, state, flags, row_cap, desc, device=0, max_launches=64, gr
         cur_state = out["state"][:, again]
         cur_flags = out["flags"][again]
         cur_cap = np.maximum(16, (cur_cap[again] * grow).astype(np.int64))
-    rows = [np.concatenate(r) if r else np.zeros((0, width)) for r in rows]
     return TraceResult(rows, final_state, final_flags, status, naccpt, tot, launches)
 
 

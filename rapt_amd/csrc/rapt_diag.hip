@@ -25,14 +25,13 @@ extern "C" int rapt_particle_gc(rapt_ctx* c, int64_t n, const double* rows, cons
   if (n == 0) return RAPT_OK;
   HIP_OK(c, hipSetDevice(c->device));
   const int64_t nmq = per_row ? n : 1;
-  double *d_rows = nullptr, *d_m = nullptr, *d_q = nullptr, *d_out = nullptr;
-  int32_t* d_st = nullptr;
+  Workspace ws(c);
+  double* d_rows = (double*)ws.get((size_t)n * (13 * sizeof(double) + sizeof(int32_t)) +
+                                   2 * sizeof(double) * nmq);
+  double *d_m = d_rows + 7 * n, *d_q = d_m + nmq, *d_out = d_q + nmq;
+  int32_t* d_st = (int32_t*)(d_out + 6 * n);
   int rc = RAPT_OK;
-  if (hipMalloc(&d_rows, sizeof(double) * 7 * n) != hipSuccess ||
-      hipMalloc(&d_m, sizeof(double) * nmq) != hipSuccess ||
-      hipMalloc(&d_q, sizeof(double) * nmq) != hipSuccess ||
-      hipMalloc(&d_out, sizeof(double) * 6 * n) != hipSuccess ||
-      hipMalloc(&d_st, sizeof(int32_t) * n) != hipSuccess) {
+  if (!d_rows) {
     rc = set_err(c, RAPT_E_OOM, "diagnostics allocation failed");
   } else if (hipMemcpyAsync(d_rows, rows, sizeof(double) * 7 * n, hipMemcpyHostToDevice,
                             c->stream) != hipSuccess ||
@@ -78,17 +77,11 @@ extern "C" int rapt_particle_gc(rapt_ctx* c, int64_t n, const double* rows, cons
     }
     if (rc == RAPT_OK &&
         (hipGetLastError() != hipSuccess ||
-         hipMemcpyAsync(out, d_out, sizeof(double) * 6 * n, hipMemcpyDeviceToHost, c->stream) !=
-             hipSuccess ||
+         rapt_copy_out(c, out, d_out, sizeof(double) * 6 * n) != hipSuccess ||
          hipMemcpyAsync(status, d_st, sizeof(int32_t) * n, hipMemcpyDeviceToHost, c->stream) !=
              hipSuccess ||
          hipStreamSynchronize(c->stream) != hipSuccess))
       rc = set_err(c, RAPT_E_HIP, "diagnostics kernel failed");
   }
-  (void)hipFree(d_rows);
-  (void)hipFree(d_m);
-  (void)hipFree(d_q);
-  (void)hipFree(d_out);
-  (void)hipFree(d_st);
   return rc;
 }

@@ -22,6 +22,8 @@
 #define RAPT_JIT_RHS_EVAL 17
 #define RAPT_JIT_PARTICLE_GC 18
 
+#define RAPT_RING_SLOTS 8  // slots of the pinned ring (rapt_copy.hip)
+
 // Grid of a lane-group GuidingCenter launch: single layouts (L = 2, 4, 8)
 // `groups` resident groups of L lanes; mixed layouts (lanes_per_particle 3,
 // 5) `groups` octets, `quads` quads and `pairs` pairs, whose blocks are
@@ -65,11 +67,15 @@ struct rapt_ctx {
   // device address of this device's allocation-free scratch (the work-queue
   // and step counters of rapt_trace_device_noalloc), from hipGetSymbolAddress
   unsigned long long* noalloc_scratch = nullptr;
-  // device scratch of the field-line entry points, kept between calls
-  // (Workspace below)
+  // device scratch of the entry points that take and return host arrays, kept
+  // between calls (Workspace below)
   std::mutex ws_mu;
   void* ws = nullptr;
   size_t ws_bytes = 0;
+  // pinned ring of rapt_copy_out, made by the first large copy
+  std::mutex ring_mu;
+  char* ring = nullptr;
+  hipEvent_t ring_ev[RAPT_RING_SLOTS] = {};
   std::string err;
 };
 
@@ -128,6 +134,11 @@ static inline hipError_t ctx_malloc(rapt_ctx* c, void** p, size_t bytes) {
   }
   return e;
 }
+
+// Copies device memory to host memory on the context's stream, as hipMemcpyAsync
+// does: dst is complete once the stream is synchronised (rapt_copy.hip).
+hipError_t rapt_copy_out(rapt_ctx* c, void* dst, const void* src, size_t bytes);
+void rapt_ring_free(rapt_ctx* c);
 
 // run-time compiled tracer kernels of a user-written field (rapt_jit.hip)
 int rapt_jit_prepare(rapt_ctx* c, int kind, bool sp);

@@ -813,6 +813,76 @@ static TrainArgs train_args(const rapt_mlp* m, int bt) {
   return A;
 }
 
+// Values in double precision, the drift's sign applied
+__global__ void k_widen(int64_t n, const float* v, double sign, double* out) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = i % 3 == 1 ? (double)v[i] * sign : (double)v[i];
+}
+
+// rapt_mlp_infer (out) and rapt_mlp_infer_values (wide)
+static int infer(rapt_mlp* m, int64_t n, const float* query, float thresh, float* out,
+                 double* wide, double sign, int32_t* flag, float* raw, double* kernel_ms) {
+  rapt_ctx* c = m->ctx;
+  HIP_OK(c, hipSetDevice(c->device));
+  hipStream_t st = c->stream;
+  if (!m->packed_ok) {
+    for (int layer = 0; layer < 2; ++layer)
+      hipLaunchKernelGGL(k_pack, dim3(PACKED / 256, 1, m->members), dim3(256), 0, st, m->wb,
+                         m->packed + (int64_t)layer * PACKED, layer == 0 ? OFF_W2 : OFF_W3);
+    hipLaunchKernelGGL(k_pack1, dim3(P1SIZE / 256, 1, m->members), dim3(256), 0, st, m->wb,
+                       m->p1);
+    HIP_OK(c, hipGetLastError());
+    m->packed_ok = true;
+  }
+  Workspace ws(c);
+  const size_t nraw = raw ? (size_t)3 * n * m->members : 0;
+  // (read in fours: at the front)
+  float* dprep = (float*)ws.get(sizeof(double) * (wide ? 3 * n : 0) +
+                                sizeof(float) * (15 * n + nraw));
+  if (!dprep) return set_err(c, RAPT_E_OOM, "inference allocation failed");
+  double* dwide = (double*)(dprep + 8 * n);
+  float* dq = (float*)(dwide + (wide ? 3 * n : 0));
+  float *dout = dq + 3 * n, *draw = dout + 3 * n;
+  int32_t* dflag = (int32_t*)(draw + nraw);
+  HIP_OK(c, hipMemcpyAsync(dq, query, sizeof(float) * 3 * n, hipMemcpyHostToDevice, st));
+  InferArgs A;
+  A.n = n;
+  A.members = m->members;
+  A.wb = m->wb;
+  A.packed = m->packed;
+  A.p1 = m->p1;
+  A.norm = m->norm;
+  A.thresh = thresh;
+  A.prep = dprep;
+  A.out = dout;
+  A.raw = raw ? draw : nullptr;
+  A.flag = dflag;
+  int dev_cus = 256;
+  (void)hipDeviceGetAttribute(&dev_cus, hipDeviceAttributeMultiprocessorCount, c->device);
+  HIP_OK(c, hipEventRecord(c->ev0, st));
+  hipLaunchKernelGGL(k_prep, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, dq,
+                     m->split, m->mass, m->eV, dprep, dflag);
+  rapt_launch_infer(st, A, dev_cus);
+  HIP_OK(c, hipEventRecord(c->ev1, st));
+  if (wide)
+    hipLaunchKernelGGL(k_widen, dim3((unsigned)((3 * n + 255) / 256)), dim3(256), 0, st, 3 * n,
+                       dout, sign, dwide);
+  if (hipGetLastError() != hipSuccess ||
+      (out && rapt_copy_out(c, out, dout, sizeof(float) * 3 * n) != hipSuccess) ||
+      (wide && rapt_copy_out(c, wide, dwide, sizeof(double) * 3 * n) != hipSuccess) ||
+      hipMemcpyAsync(flag, dflag, sizeof(int32_t) * n, hipMemcpyDeviceToHost, st) !=
+          hipSuccess ||
+      (raw && rapt_copy_out(c, raw, draw, sizeof(float) * nraw) != hipSuccess) ||
+      hipStreamSynchronize(st) != hipSuccess)
+    return set_err(c, RAPT_E_HIP, "inference kernel failed");
+  if (kernel_ms) {
+    float ms = 0.0f;
+    (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
+    *kernel_ms = ms;
+  }
+  return RAPT_OK;
+}
+
 extern "C" {
 
 int rapt_mlp_create(rapt_ctx* c, int32_t members, const float* theta0, double mass, double eV,
@@ -1069,71 +1139,14 @@ int rapt_mlp_infer(rapt_mlp* m, int64_t n, const float* query, float thresh, flo
                    int32_t* flag, float* raw, double* kernel_ms) {
   if (!m || n <= 0 || !query || !out || !flag)
     return m ? set_err(m->ctx, RAPT_E_ARG, "bad infer call") : RAPT_E_ARG;
-  rapt_ctx* c = m->ctx;
-  HIP_OK(c, hipSetDevice(c->device));
-  hipStream_t st = c->stream;
-  if (!m->packed_ok) {
-    for (int layer = 0; layer < 2; ++layer)
-      hipLaunchKernelGGL(k_pack, dim3(PACKED / 256, 1, m->members), dim3(256), 0, st, m->wb,
-                         m->packed + (int64_t)layer * PACKED, layer == 0 ? OFF_W2 : OFF_W3);
-    hipLaunchKernelGGL(k_pack1, dim3(P1SIZE / 256, 1, m->members), dim3(256), 0, st, m->wb,
-                       m->p1);
-    HIP_OK(c, hipGetLastError());
-    m->packed_ok = true;
-  }
-  float *dq = nullptr, *dout = nullptr, *draw = nullptr, *dprep = nullptr;
-  int32_t* dflag = nullptr;
-  int rc = RAPT_OK;
-  if (hipMalloc(&dq, sizeof(float) * 3 * n) != hipSuccess ||
-      hipMalloc(&dprep, sizeof(float) * 8 * n) != hipSuccess ||
-      hipMalloc(&dout, sizeof(float) * 3 * n) != hipSuccess ||
-      hipMalloc(&dflag, sizeof(int32_t) * n) != hipSuccess ||
-      (raw && hipMalloc(&draw, sizeof(float) * 3 * n * m->members) != hipSuccess)) {
-    rc = set_err(c, RAPT_E_OOM, "inference allocation failed");
-  } else if (hipMemcpyAsync(dq, query, sizeof(float) * 3 * n, hipMemcpyHostToDevice, st) !=
-             hipSuccess) {
-    rc = set_err(c, RAPT_E_HIP, "query copy failed");
-  } else {
-    InferArgs A;
-    A.n = n;
-    A.members = m->members;
-    A.wb = m->wb;
-    A.packed = m->packed;
-    A.p1 = m->p1;
-    A.norm = m->norm;
-    A.thresh = thresh;
-    A.prep = dprep;
-    A.out = dout;
-    A.raw = draw;
-    A.flag = dflag;
-    int dev_cus = 256;
-    (void)hipDeviceGetAttribute(&dev_cus, hipDeviceAttributeMultiprocessorCount, c->device);
-    HIP_OK(c, hipEventRecord(c->ev0, st));
-    hipLaunchKernelGGL(k_prep, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, dq,
-                       m->split, m->mass, m->eV, dprep, dflag);
-    rapt_launch_infer(st, A, dev_cus);
-    HIP_OK(c, hipEventRecord(c->ev1, st));
-    if (hipGetLastError() != hipSuccess ||
-        hipMemcpyAsync(out, dout, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, st) !=
-            hipSuccess ||
-        hipMemcpyAsync(flag, dflag, sizeof(int32_t) * n, hipMemcpyDeviceToHost, st) !=
-            hipSuccess ||
-        (raw && hipMemcpyAsync(raw, draw, sizeof(float) * 3 * n * m->members,
-                               hipMemcpyDeviceToHost, st) != hipSuccess) ||
-        hipStreamSynchronize(st) != hipSuccess) {
-      rc = set_err(c, RAPT_E_HIP, "inference kernel failed");
-    } else if (kernel_ms) {
-      float ms = 0.0f;
-      (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
-      *kernel_ms = ms;
-    }
-  }
-  (void)hipFree(dq);
-  (void)hipFree(dprep);
-  (void)hipFree(dout);
-  (void)hipFree(dflag);
-  (void)hipFree(draw);
-  return rc;
+  return infer(m, n, query, thresh, out, nullptr, 1.0, flag, raw, kernel_ms);
+}
+
+int rapt_mlp_infer_values(rapt_mlp* m, int64_t n, const float* query, float thresh, double sign,
+                          double* out, int32_t* flag, float* raw, double* kernel_ms) {
+  if (!m || n <= 0 || !query || !out || !flag)
+    return m ? set_err(m->ctx, RAPT_E_ARG, "bad infer call") : RAPT_E_ARG;
+  return infer(m, n, query, thresh, nullptr, out, sign, flag, raw, kernel_ms);
 }
 
 }  // extern "C"

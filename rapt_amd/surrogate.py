@@ -168,15 +168,15 @@ class Surrogate:
         outputs or None, kernel ms)."""
         q = np.ascontiguousarray(query, np.float32)
         n = q.shape[0]
-        out = np.zeros((n, 3), np.float32)
+        out = np.zeros((n, 3))
         flag = np.zeros(n, np.int32)
         rw = np.zeros((self.members, n, 3), np.float32) if raw else None
         ms = C.c_double(0.0)
-        self.ctx.check(N.lib().rapt_mlp_infer(self.h, n, _fp(q), thresh, _fp(out),
-                                              N._ip32(flag), _fp(rw) if raw else None,
-                                              C.byref(ms)), "rapt_mlp_infer")
-        out = out.astype(np.float64)
-        out[:, 1] *= -np.sign(self.charge)   # positive charges drift westward
+        # (positive charges drift westward)
+        self.ctx.check(N.lib().rapt_mlp_infer_values(self.h, n, _fp(q), thresh,
+                                                     -np.sign(self.charge), N._dp(out),
+                                                     N._ip32(flag), _fp(rw) if raw else None,
+                                                     C.byref(ms)), "rapt_mlp_infer_values")
         return out, flag, rw, ms.value
 
     def predict(self, query, thresh=1e-3, params=None):

@@ -1,0 +1,52 @@
+"""Results large enough for the staged copies (rapt_copy.hip), a megabyte a
+slot of a ring of eight: one slot short of the threshold, at it, a last slot
+that is not full, the ring more than once round; and from two threads at once."""
+import threading
+
+import numpy as np
+import pytest
+
+from rapt_amd import _native as N
+from rapt_amd import constants as K
+from rapt_amd import fields as F
+
+pytestmark = pytest.mark.gpu
+
+MB = 1 << 20
+
+
+def _points(n):
+    rng = np.random.default_rng(n)
+    return np.c_[np.zeros(n), rng.uniform(2, 8, (n, 3)) * K.Re]
+
+
+@pytest.mark.parametrize("nbytes", [4 * MB - 8, 4 * MB, 4 * MB + 8, 8 * MB, 21 * MB + 1000])
+def test_large_results_equal_small_ones(nbytes):
+    f = F.EarthDipole().descriptor()
+    ctx = N.context()
+    tp = _points(nbytes // 8)
+    got = ctx.field_eval(f, "magB", tp)
+    step = 100000
+    ref = np.concatenate([ctx.field_eval(f, "magB", tp[i:i + step])
+                          for i in range(0, len(tp), step)])
+    np.testing.assert_array_equal(got, ref)
+
+
+def test_large_results_on_two_threads():
+    f = F.EarthDipole().descriptor()
+    ctx = N.context()
+    tp = [_points(700001), _points(900003)]
+    ref = [ctx.field_eval(f, "B", t) for t in tp]
+    got = [None, None]
+
+    def work(i):
+        for _ in range(3):
+            got[i] = ctx.field_eval(f, "B", tp[i])
+
+    th = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    for g, r in zip(got, ref):
+        np.testing.assert_array_equal(g, r)
