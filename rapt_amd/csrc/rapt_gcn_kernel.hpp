@@ -19,8 +19,11 @@
 //
 // For a time-dependent field lane 0's spare evaluation (lane 7's for L = 8)
 // is the centre at t - tstep.  Each lane forms its share of grad|B| and
-// curl b, the shares are broadcast back, and every lane runs the shared
-// guiding-centre algebra and keeps its own output components.  All
+// curl b, the shares are broadcast back (a broadcast names the lane that it
+// reads, so each quantity is read from its own register: collecting a lane's
+// shares in common registers first took 10-12 selects a right-hand side, 3-5%
+// of an advance), and every lane runs the shared guiding-centre algebra and
+// keeps its own output components.  All
 // reductions (error norm, HINIT norms) are summed in one fixed order from
 // broadcast values, so the lanes of a group stay bit-identical, take the
 // same branches, and the trajectories are bit-identical to the one-lane
@@ -229,16 +232,13 @@ __device__ __forceinline__ CV<1> rhs_gc_quad(const FieldC& F, int eom, bool stat
   mag_unit(Bb, mb, ub_);
   const V3 du{ua.x - ub_.x, ua.y - ub_.y, ua.z - ub_.z};
   const double g = (ma - mb) * i2d;
-  const double e0 = (q == 0) ? Ba.x : g;
-  const double e1 = (q == 0) ? Ba.y : ((q == 1) ? du.y : du.x);
-  const double e2 = (q == 0) ? Ba.z : ((q == 3) ? du.y : du.z);
-  const V3 B{gb<4, 0>(e0), gb<4, 0>(e1), gb<4, 0>(e2)};
+  const V3 B{gb<4, 0>(Ba.x), gb<4, 0>(Ba.y), gb<4, 0>(Ba.z)};
   // |B| and b at the centre: lane 0's own mag_unit of Ba
   const double Bm = gb<4, 0>(ma);
   const V3 ub{gb<4, 0>(ua.x), gb<4, 0>(ua.y), gb<4, 0>(ua.z)};
-  const V3 gB{gb<4, 1>(e0), gb<4, 2>(e0), gb<4, 3>(e0)};
-  const V3 cb = curl_from_pairs(gb<4, 1>(e1), gb<4, 1>(e2), gb<4, 2>(e1), gb<4, 2>(e2),
-                                gb<4, 3>(e1), gb<4, 3>(e2), i2d);
+  const V3 gB{gb<4, 1>(g), gb<4, 2>(g), gb<4, 3>(g)};
+  const V3 cb = curl_from_pairs(gb<4, 1>(du.y), gb<4, 1>(du.z), gb<4, 2>(du.x), gb<4, 2>(du.z),
+                                gb<4, 3>(du.x), gb<4, 3>(du.y), i2d);
   V3 db{0.0, 0.0, 0.0};
   if (eom == EOM_TCB && !stat) {
     // lane 0's second point was B(t - tstep); B(t + tstep) is a third evaluation
@@ -281,21 +281,16 @@ __device__ __forceinline__ CV<2> rhs_gc_pair(const FieldC& F, int eom, bool stat
   mag_unit(B1, m1, u1);
   mag_unit(B2, m2, u2);
   mag_unit(B3, m3, u3);
-  // lane 0 sends (B, d|B|/dx, dxy, dxz); lane 1 sends (d|B|/dy, d|B|/dz,
-  // dyx, dyz, dzx, dzy), where dxy = b_y(+x) - b_y(-x) and so on
-  const double e0 = l0 ? B0.x : (m0 - m1) * i2d;
-  const double e1 = l0 ? B0.y : (m2 - m3) * i2d;
-  const double e2 = l0 ? B0.z : u0.x - u1.x;
-  const double e3 = l0 ? (m1 - m2) * i2d : u0.z - u1.z;
-  const double e4 = l0 ? u1.y - u2.y : u2.x - u3.x;
-  const double e5 = l0 ? u1.z - u2.z : u2.y - u3.y;
-  const V3 B{gb<2, 0>(e0), gb<2, 0>(e1), gb<2, 0>(e2)};
+  // lane 0 sends (B, d|B|/dx, dxy, dxz), lane 1 (d|B|/dy, d|B|/dz, dyx, dyz,
+  // dzx, dzy), where dxy = b_y(+x) - b_y(-x) and so on
+  const V3 B{gb<2, 0>(B0.x), gb<2, 0>(B0.y), gb<2, 0>(B0.z)};
   // |B| and b at the centre: lane 0's own mag_unit of B0
   const double Bm = gb<2, 0>(m0);
   const V3 ub{gb<2, 0>(u0.x), gb<2, 0>(u0.y), gb<2, 0>(u0.z)};
-  const V3 gB{gb<2, 0>(e3), gb<2, 1>(e0), gb<2, 1>(e1)};
-  const V3 cb = curl_from_pairs(gb<2, 0>(e4), gb<2, 0>(e5), gb<2, 1>(e2), gb<2, 1>(e3),
-                                gb<2, 1>(e4), gb<2, 1>(e5), i2d);
+  const V3 gB{gb<2, 0>((m1 - m2) * i2d), gb<2, 1>((m0 - m1) * i2d), gb<2, 1>((m2 - m3) * i2d)};
+  const V3 cb = curl_from_pairs(gb<2, 0>(u1.y - u2.y), gb<2, 0>(u1.z - u2.z),
+                                gb<2, 1>(u0.x - u1.x), gb<2, 1>(u0.z - u1.z),
+                                gb<2, 1>(u2.x - u3.x), gb<2, 1>(u2.y - u3.y), i2d);
   V3 db{0.0, 0.0, 0.0};
   if (eom == EOM_TCB && !stat) {
     // lane 0's fourth point was B(t - tstep); B(t + tstep) is a fifth evaluation
@@ -340,15 +335,12 @@ __device__ __forceinline__ CV<1> rhs_gc_oct(const FieldC& F, int eom, bool stat,
   const V3 ub_{gmir(ua.x), gmir(ua.y), gmir(ua.z)};
   const V3 du{ua.x - ub_.x, ua.y - ub_.y, ua.z - ub_.z};
   const double g = (ma - mb) * i2d;
-  const double e0 = (q == 0) ? Ba.x : g;
-  const double e1 = (q == 0) ? Ba.y : ((q == 1) ? du.y : du.x);
-  const double e2 = (q == 0) ? Ba.z : ((q == 3) ? du.y : du.z);
-  const V3 B{gb<4, 0>(e0), gb<4, 0>(e1), gb<4, 0>(e2)};
+  const V3 B{gb<4, 0>(Ba.x), gb<4, 0>(Ba.y), gb<4, 0>(Ba.z)};
   const double Bm = gb<4, 0>(ma);
   const V3 ub{gb<4, 0>(ua.x), gb<4, 0>(ua.y), gb<4, 0>(ua.z)};
-  const V3 gB{gb<4, 1>(e0), gb<4, 2>(e0), gb<4, 3>(e0)};
-  const V3 cb = curl_from_pairs(gb<4, 1>(e1), gb<4, 1>(e2), gb<4, 2>(e1), gb<4, 2>(e2),
-                                gb<4, 3>(e1), gb<4, 3>(e2), i2d);
+  const V3 gB{gb<4, 1>(g), gb<4, 2>(g), gb<4, 3>(g)};
+  const V3 cb = curl_from_pairs(gb<4, 1>(du.y), gb<4, 1>(du.z), gb<4, 2>(du.x), gb<4, 2>(du.z),
+                                gb<4, 3>(du.x), gb<4, 3>(du.y), i2d);
   V3 db{0.0, 0.0, 0.0};
   if (eom == EOM_TCB && !stat) {
     // lane 0's partner point was B(t - tstep); B(t + tstep) is a second evaluation

@@ -793,7 +793,8 @@ static int spread_lanes(int64_t n, int64_t waves) {
 // SIMD, each lane group taking particles from the queue, ends sooner than two
 // that slow each other down and have nothing to refill from.  `one` lanes are a
 // wave a SIMD (65,536).  DoubleDipole electrons, advance(10), output step 1 s,
-// quads all resident as before, then this layout, ms:
+// quads all resident as before, then this layout, ms (every layout has become 3-5%
+// faster since):
 //   octets, one wave a SIMD, up to `one` / 4:  10,000 14.5, 12.4; 16,384 14.7, 12.9
 //   quads, one wave a SIMD, up to `one` / 2:   24,576 17.0, 15.1; 32,768 18.4, 15.2
 //   pairs and, for the costliest, quads (as many as fit beside the pairs' chains:
