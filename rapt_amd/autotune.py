@@ -48,6 +48,18 @@ def candidates(mode, stepper, precision, n):
                             mixed_quads=max(1, n // frac)))
         out.append(dict(lanes_per_particle=5, block=256, lanes=0,
                         mixed_octets=max(1, n // 128), mixed_quads=max(1, n // 8)))
+        # one wave a SIMD (65,536 lanes), refilled from the queue: the longest
+        # traces' waves share their SIMD with no other (65,536 DoubleDipole
+        # electrons, advance(60): 121 ms against 127-137 with every lane
+        # resident, 512 octets and 8,192 quads in front); two where there are
+        # enough particles to even out
+        if 8192 < n <= 32768:
+            out.append(dict(lanes_per_particle=8 if n <= 16384 else 4, block=64, lanes=65536))
+        elif 32768 < n <= 131072:
+            for quads in (2048, 4096):
+                out.append(dict(lanes_per_particle=3, block=64, lanes=65536, mixed_quads=quads))
+        if n > 65536:
+            out.append(dict(lanes_per_particle=3, block=64, lanes=2 * 65536, mixed_quads=1))
     # fewer resident lanes than particles: refill from the queue sooner
     if n >= 8 * 65536:
         out.append(dict(lanes_per_particle=1, block=256, lanes=4 * 65536))
