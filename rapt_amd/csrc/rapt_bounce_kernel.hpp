@@ -43,10 +43,10 @@
 // issue (127,000 instructions a wave of 32 lines) and the points' traffic.
 // Against one lane a line, with a binary search through the scratch, a cosine
 // and a sine at each of the 512 nodes, a |B| evaluation beside each point's
-// direction and 16,384 lanes at most: S_b of 65,536 lines 12.1 -> 0.81 ms,
+// direction and 16,384 lanes at most: S_b of 65,536 lines 12.1 -> 0.80 ms,
 // labels 17.0 -> 1.2 ms (16,384 queries; 10.1 on the 72 waves they are launched
 // with, rapt_bounce.hip) and 14.8 -> 0.46 ms (300), five bounce centres over four
-// rows 400 -> 11.5 ms, the same results bit for bit.
+// rows 400 -> 11.1 ms, the same results bit for bit.
 #pragma once
 #ifndef __HIPCC_RTC__
 #include <hip/hip_runtime.h>
