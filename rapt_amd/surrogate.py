@@ -168,15 +168,25 @@ class Surrogate:
         outputs or None, kernel ms)."""
         q = np.ascontiguousarray(query, np.float32)
         n = q.shape[0]
-        out = np.zeros((n, 3))
         flag = np.zeros(n, np.int32)
         rw = np.zeros((self.members, n, 3), np.float32) if raw else None
         ms = C.c_double(0.0)
-        # (positive charges drift westward)
-        self.ctx.check(N.lib().rapt_mlp_infer_values(self.h, n, _fp(q), thresh,
-                                                     -np.sign(self.charge), N._dp(out),
-                                                     N._ip32(flag), _fp(rw) if raw else None,
-                                                     C.byref(ms)), "rapt_mlp_infer_values")
+        sign = -np.sign(self.charge)   # positive charges drift westward
+        # The device widens large results (524,288 queries 1.5 ms, widened here
+        # 3.1; 262,144 0.82 and 0.84); its launch and the wider copy cost more
+        # than they save on small ones (131,072 0.52 and 0.45, 1,000 0.14 and 0.11)
+        if n >= 1 << 18:
+            out = np.zeros((n, 3))
+            self.ctx.check(N.lib().rapt_mlp_infer_values(
+                self.h, n, _fp(q), thresh, sign, N._dp(out), N._ip32(flag),
+                _fp(rw) if raw else None, C.byref(ms)), "rapt_mlp_infer_values")
+            return out, flag, rw, ms.value
+        out = np.zeros((n, 3), np.float32)
+        self.ctx.check(N.lib().rapt_mlp_infer(self.h, n, _fp(q), thresh, _fp(out),
+                                              N._ip32(flag), _fp(rw) if raw else None,
+                                              C.byref(ms)), "rapt_mlp_infer")
+        out = out.astype(np.float64)
+        out[:, 1] *= sign
         return out, flag, rw, ms.value
 
     def predict(self, query, thresh=1e-3, params=None):

@@ -50,3 +50,19 @@ def test_large_results_on_two_threads():
         t.join()
     for g, r in zip(got, ref):
         np.testing.assert_array_equal(g, r)
+
+
+def test_inference_values_on_either_side_of_the_device_widening():
+    """From 262,144 queries on the device widens the values and applies the
+    drift's sign: the bits of the float path."""
+    from rapt_amd import surrogate as S
+    rng = np.random.default_rng(4)
+    n = 1 << 18
+    q = np.c_[rng.uniform(2, 8, n), rng.uniform(10, 89, n), rng.uniform(4, 7, n)]
+    for charge in (K.e, -K.e):
+        s = S.Surrogate(F.EarthDipole(), charge=charge, members=2, seed=1)
+        v, flag, raw, _ = s.infer(q, raw=True)
+        a, b = s.infer(q[:-1], raw=True), s.infer(q[-1:], raw=True)
+        np.testing.assert_array_equal(v, np.r_[a[0], b[0]])
+        np.testing.assert_array_equal(flag, np.r_[a[1], b[1]])
+        np.testing.assert_array_equal(raw, np.concatenate([a[2], b[2]], axis=1))
