@@ -44,22 +44,28 @@ static void launch_order(rapt_ctx* c, const BounceArgs& A, bool labels, int32_t*
 // the call repeated with CAP_MOST and 16,384 lines in the same memory.
 static constexpr int32_t CAP_FIRST = 512, CAP_MOST = 2048;
 
-// Waves of a surrogate-label launch.  The labels are the yardstick of the
-// surrogate, whose inference kernel is held to at least 300 times their rate on
-// 65,536 queries (tests/test_gpu_surrogate.py): with every wave resident they
-// take 5.2 ms, 50 times the ensemble's 0.106 ms.  72 waves: 65,536 queries
-// 38-42 ms, 350-400 times (80 waves 330-365, 96 280-315); 16,384 in 10.3 ms and
-// 300, which fit into them, in 0.5 (a lane a line, every line resident: 17.8 and
-// 14.9); 16,384 with every wave resident 1.2.
+// Waves of a surrogate-label launch in a dipole-type field.  No resource asks
+// for this limit: with every wave resident 65,536 queries take 5.2 ms and
+// 16,384 1.2, with it 38-42 and 10.3 (300 queries, which fit, 0.5).  It holds
+// the labels to what the ensemble's inference, 0.106 ms for 65,536 queries, is
+// tested to be 300 times faster than (tests/test_gpu_surrogate.py), a bar that
+// was set when a lane traced a query's lines, every query resident, and 65,536
+// took 67 ms; they are not slower than that.  They would be where a line costs
+// more beside its quadrature, so those launches have no limit: gridded and
+// user-written fields (16,384 queries, ms, that kernel / 72 waves / no limit:
+// grid 18.3, 17.9, 2.2; compiled 18.8, 19.5, 1.6; interpreted 95.6, 203, 18.4), and the
+// second attempt of lines too long for the first (dipole plus uniform at
+// fieldlineresolution 200: 46.3, 52.9, 32.3).
 static constexpr int64_t LABEL_WAVES = 72;
 
-// Fills in the resident work items, the scratch strides and the scratch
-// itself; items of five lines (groups) or one.  Returns the grid, or 0 when
-// the scratch does not fit.
+// Fills in the resident work items (on `waves` waves at most, 0: as many as the
+// scratch has points for), the scratch strides and the scratch itself; items
+// of five lines (groups) or one.  Returns the grid, or 0 when the scratch does
+// not fit.
 static unsigned bounce_scratch(Workspace& ws, BounceArgs& A, int64_t n, int32_t cap, bool groups,
-                               bool positions, size_t extra, char** extra_mem) {
+                               bool positions, int64_t waves, size_t extra, char** extra_mem) {
   int64_t most = (int64_t)2048 * CAP_FIRST / cap;  // resident waves
-  if (positions && most > LABEL_WAVES) most = LABEL_WAVES;
+  if (waves > 0 && most > waves) most = waves;
   const int64_t per_wave = groups ? GRP_PER_WAVE : 32;
   int64_t blocks = (n + per_wave - 1) / per_wave;
   if (blocks > most) blocks = most;
@@ -109,7 +115,10 @@ static int run_bounce(rapt_ctx* c, int64_t n, const double* in, int in_w, const 
   const size_t doubles = (size_t)n * (in_w + (Bm ? 1 : 0) + out_w);
   for (int32_t cap = CAP_FIRST;; cap = CAP_MOST) {
     char* mem = nullptr;
+    const int m = c->field.model;
+    const bool limit = lab && cap == CAP_FIRST && m != RAPT_FIELD_GRID && m != RAPT_FIELD_EXPR;
     const unsigned grid = bounce_scratch(ws, A, n, cap, lab != nullptr, positions,
+                                         limit ? LABEL_WAVES : 0,
                                          sizeof(double) * doubles + sizeof(int32_t) * 2 * n, &mem);
     if (!grid) return set_err(c, RAPT_E_OOM, "bounce scratch allocation failed");
     double* d_in = (double*)mem;
@@ -261,7 +270,7 @@ extern "C" int rapt_bounce_center_advance(rapt_ctx* c, int64_t n, double* tpos, 
   const size_t bytes = 8 * (8 * (size_t)n + rows_w + 3 * (size_t)n) + sizeof(int32_t) * n;
   for (int32_t cap = CAP_FIRST;; cap = CAP_MOST) {
     char* mem = nullptr;
-    const unsigned grid = bounce_scratch(ws, A, n, cap, true, false, bytes, &mem);
+    const unsigned grid = bounce_scratch(ws, A, n, cap, true, false, 0, bytes, &mem);
     if (!grid) return set_err(c, RAPT_E_OOM, "BounceCenter allocation failed");
     double* d_tpos = (double*)mem;
     double* d_in = d_tpos + 4 * n;
