@@ -74,6 +74,7 @@ using namespace rapt;
 struct rapt_batch {
   rapt_ctx* ctx = nullptr;
   int64_t n = 0;
+  double costly = 0.0;  // of the uploaded particles (default_layout)
   char* mem = nullptr;  // one allocation for d_state .. d_order and d_work
   double* d_state = nullptr;
   double* d_state0 = nullptr;  // state as uploaded (rapt_batch_reset)
@@ -133,6 +134,13 @@ static std::vector<int64_t> sorted_items(std::vector<WorkKey>& key) {
   std::vector<int64_t> items(key.size());
   for (size_t i = 0; i < key.size(); ++i) items[i] = key[i].item;
   return items;
+}
+
+// Particles that cost as much as the costliest, of the same sum: n where
+// nothing is known of their costs.
+static double costly(int64_t n, double sum, double most) {
+  const double k = sum / most;
+  return k >= 1.0 && k <= (double)n ? k : (double)n;
 }
 
 static int field_width(int what) {
@@ -675,6 +683,7 @@ int rapt_batch_upload(rapt_batch* b, const double* state, const int32_t* flags) 
   const double* dts = state + (size_t)RAPT_S_DT * b->n;
   const double* v = state + (size_t)RAPT_S_V * b->n;
   const double* y = state + (size_t)RAPT_S_Y0 * b->n;
+  double sum = 0.0, most = 0.0;  // of the steps that the particles may need
   bool equal = dts[0] > 0.0;
   for (int64_t i = 1; i < b->n && equal; ++i) equal = dts[i] == dts[0];
   try {
@@ -686,9 +695,13 @@ int rapt_batch_upload(rapt_batch* b, const double* state, const int32_t* flags) 
         k = sqrt(*yx * *yx + *yy * *yy + *yz * *yz) / v[i];
       }
       if (!(k > 0.0)) k = HUGE_VAL;  // (no step, no speed, not a number: last)
+      const double cost = 1.0 / k;
+      sum += cost;
+      most = cost > most ? cost : most;
       key[(size_t)i].item = i;
       memcpy(&key[(size_t)i].bits, &k, sizeof k);
     }
+    b->costly = costly(b->n, sum, most);
     const std::vector<int64_t> order = sorted_items(key);
     HIP_OK(c, hipMemcpyAsync(b->d_order, order.data(), sizeof(int64_t) * b->n,
                              hipMemcpyHostToDevice, c->stream));
@@ -711,6 +724,12 @@ int rapt_batch_set_cost(rapt_batch* b, const double* cost) {
   for (int64_t i = 0; i < b->n; ++i) order[(size_t)i] = i;
   std::stable_sort(order.begin(), order.end(),
                    [cost](int64_t a, int64_t q) { return cost[a] > cost[q]; });
+  double sum = 0.0, most = 0.0;
+  for (int64_t i = 0; i < b->n; ++i) {
+    sum += cost[i] > 0.0 ? cost[i] : 0.0;
+    most = cost[i] > most ? cost[i] : most;
+  }
+  b->costly = costly(b->n, sum, most);
   HIP_OK(c, hipMemcpyAsync(b->d_order, order.data(), sizeof(int64_t) * b->n,
                            hipMemcpyHostToDevice, c->stream));
   HIP_OK(c, hipStreamSynchronize(c->stream));
@@ -802,36 +821,62 @@ static int spread_lanes(int64_t n, int64_t waves) {
 //                       40,000 19.3, 15.2; 65,536 22.4, 18.4; 98,304 29.1, 26.3
 //   pairs, two waves a SIMD (each has particles enough to even out):
 //            131,072 36.4, 31.4; 262,144 69.7, 55.8; 524,288 136, 105
-// and the same way in the dipole, and with output steps of a bounce period.  In
-// input order the front of the queue is not the costliest, and a gridded field
-// waits for memory, which a second wave hides: quads there (65,536: 21.8 against
-// 22.6, and 45 against 83 on a grid), octets for few (8,192 10.0, 8.2; a grid's
-// 16,384 29.9, 23.1).
-static void default_layout(const rapt_ctx* c, rapt_trace_desc& d, int64_t n, bool ordered) {
+// and the same way in the dipole, and with output steps of a bounce period.
+//
+// That needs particles of different length: `costly` is the sum of the
+// particles' expected costs in units of the largest, and where it is more than
+// the groups that are resident, the queue is worked off in rounds (advance(2) of
+// electrons of one energy and L, then of one energy: 16,384 octets 2.82 and 3.11,
+// quads all resident 1.89 and 2.70; 32,768 quads one wave a SIMD 3.45 and 3.72, all
+// resident 3.17 and 3.91; 65,536 quads and pairs 7.15 and 6.33, quads 6.01 and
+// 6.05, pairs two waves a SIMD 5.39 and 5.70): quads all resident there, and from
+// `one` on the two waves of pairs (131,072 9.1 and 8.8, quads 11.1 and 10.8).
+//
+// Octets that are all resident, one wave a SIMD, need no such thing.  In input
+// order the front of the queue is not the costliest, and a gridded field waits
+// for memory, which a second wave hides: quads above that, on a grid above
+// twice that (65,536: 21.8 against 22.6, and 45 against 83 on a grid; octets for
+// few: 8,192 10.0, 8.2; a grid's 16,384 29.9, 23.1).  So too in the current sheet and the
+// parabolic field, whose costs are not r / v's (65,536 in the sheet 19.3, quads
+// and pairs in that order 30.4; 16,384 16.9, octets 10.4).  A uniform field's step
+// is short and a launch's start and end most of it: quads up to `one` / 4 (four
+// rows each, 8,192 0.08, octets 0.13; 24,576 0.19, quads one wave a SIMD 0.14).
+static void default_layout(const rapt_ctx* c, rapt_trace_desc& d, int64_t n, bool ordered,
+                           double costly) {
+  const int model = c->field.model;
   if (d.mode != RAPT_MODE_GC || d.stepper != RAPT_STEP_DOPRI5 ||
       d.precision != RAPT_PREC_FP64 || d.lanes_per_particle != 0 || d.lanes > 0 ||
-      d.mixed_quads < 0 || c->field.model == RAPT_FIELD_EXPR)
+      d.mixed_quads < 0 || model == RAPT_FIELD_EXPR)
     return;
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess)
     return;
   const int64_t one = (int64_t)256 * cus;
-  const bool grid = c->field.model == RAPT_FIELD_GRID;
+  const bool uniform = model == RAPT_FIELD_ZERO || model == RAPT_FIELD_UNIFORM_BZ ||
+                       model == RAPT_FIELD_UNIFORM_CROSSED_EB;
+  const bool sheet = model == RAPT_FIELD_PARABOLIC || model == RAPT_FIELD_CURRENT_SHEET;
+  const bool grid = model == RAPT_FIELD_GRID;
   ordered = ordered && d.work_order == 0;
-  if (n <= (ordered ? one / 4 : one / 8)) {
+  const int64_t quads = (3 * one / 2 - n) / 8;  // in front of the pairs
+  d.lanes_per_particle = 4;
+  if (uniform && n <= one / 4) return;
+  if (n <= one / 8 || (ordered && n <= one / 4 && (grid || sheet || costly <= one / 8))) {
     d.lanes_per_particle = 8;
     d.lanes = one;
-  } else if (!ordered || grid) {
-    d.lanes_per_particle = 4;
+  } else if (!ordered || grid || sheet) {
     return;
-  } else if (n <= one / 2) {
-    d.lanes_per_particle = 4;
+  } else if (n <= one / 2 && costly <= one / 4) {
     d.lanes = one;
-  } else {
-    const int64_t quads = (3 * one / 2 - n) / 8;
+  } else if (n > one / 2 && quads > 0 && costly <= one / 2 - quads) {
     d.lanes_per_particle = 3;
-    d.mixed_quads = quads > 0 ? quads : 1;
-    d.lanes = quads > 0 ? one : 2 * one;
+    d.mixed_quads = quads;
+    d.lanes = one;
+  } else if (n >= one) {
+    d.lanes_per_particle = 3;
+    d.mixed_quads = 1;
+    d.lanes = 2 * one;
+  } else {
+    return;
   }
   if (d.block == 0) d.block = 64;
 }
@@ -1057,7 +1102,7 @@ int rapt_batch_run(rapt_batch* b, const rapt_trace_desc* desc, rapt_counters* cn
   rapt_ctx* c = b->ctx;
   rapt_trace_desc dd = *desc;
   const rapt_trace_desc* d = &dd;
-  default_layout(c, dd, b->n, true);
+  default_layout(c, dd, b->n, true, b->costly);
   KArgs A;
   int block = 256;
   int64_t lanes = 0;
@@ -1147,7 +1192,7 @@ int rapt_trace_device_noalloc(rapt_ctx* c, const rapt_trace_desc* d, int64_t n,
   // a user-written field: one lane per particle (compiled if an earlier run
   // loaded that kernel, else interpreted; loading a module allocates)
   if (c->field.model == RAPT_FIELD_EXPR) dd.lanes_per_particle = 1;
-  default_layout(c, dd, n, order != nullptr);
+  default_layout(c, dd, n, order != nullptr, (double)n);
   KArgs A;
   int block = 256;
   int64_t lanes = 0;
@@ -1229,7 +1274,7 @@ int rapt_batch_epochs_begin(rapt_batch* b, const rapt_trace_desc* desc,
   rapt_ctx* c = b->ctx;
   rapt_trace_desc dd = *desc;
   const rapt_trace_desc* d = &dd;
-  default_layout(c, dd, b->n, true);
+  default_layout(c, dd, b->n, true, b->costly);
   if (rows_per_epoch < 1) return set_err(c, RAPT_E_ARG, "rows_per_epoch must be >= 1");
   const int width = d->mode == RAPT_MODE_PARTICLE ? 7 : (d->mode == RAPT_MODE_GC ? 5 : 8);
   rapt_batch_epochs_end(b);

@@ -24,7 +24,7 @@ int fake_pinned_lookup;    /* 1: every host pointer is one of the runtime's */
 int fake_copies;           /* asynchronous copies */
 size_t fake_largest_copy;  /* bytes */
 const char* fake_last_kernel = "";
-unsigned fake_last_grid;
+unsigned fake_last_grid, fake_last_block;
 static hipError_t last;
 
 static hipError_t ret(hipError_t e) {
@@ -99,17 +99,18 @@ hipError_t hipStreamSynchronize(hipStream_t st) {
   return hipSuccess;
 }
 
-static void launched(const char* name, unsigned grid) {
+static void launched(const char* name, unsigned grid, unsigned block) {
   ++fake_pending;
   fake_last_kernel = name;
   fake_last_grid = grid;
+  fake_last_block = block;
 }
 hipError_t hipLaunchKernel(const void* fn, dim3 g, dim3 b, void** args, size_t sh,
                            hipStream_t st) {
-  (void)b, (void)args, (void)sh, (void)st;
+  (void)args, (void)sh, (void)st;
   for (int i = 0; i < n_kernels; ++i)
     if (kernels[i].fn == fn) {
-      launched(kernels[i].name, g.x);
+      launched(kernels[i].name, g.x, b.x);
       return hipSuccess;
     }
   return ret(hipErrorInvalidDeviceFunction);

@@ -70,7 +70,7 @@ class _Var:
 
     def __getattr__(self, name):
         t = {"fake_budget": C.c_size_t, "fake_used": C.c_size_t, "fake_largest_copy": C.c_size_t,
-             "fake_overflow_bytes": C.c_size_t, "fake_last_grid": C.c_uint,
+             "fake_overflow_bytes": C.c_size_t, "fake_last_grid": C.c_uint, "fake_last_block": C.c_uint,
              "fake_last_kernel": C.c_char_p}.get(name, C.c_int)
         return t.in_dll(self._lib, name)
 
@@ -96,6 +96,49 @@ def test_labels_fill_the_gpu(fake, name, n, attempt):
     """Labels in fields whose evaluation is most of a line, and lines too long
     for the first scratch size, run with every wave that the scratch has."""
     _run(fake, "case_labels", name, n, attempt)
+
+
+# ---- guiding-centre layouts ----------------------------------------------------------
+
+
+def case_layout(rt, name, n, costs, kernel, lanes):
+    f = {"sheet": F.CurrentSheet, "bz": F.UniformBz}[name]() if name in ("sheet", "bz") \
+        else _field(name)
+    ctx = _ctx(f)
+    S = np.zeros((N.NSLOT, n))
+    S[N.S_Y0] = 5 * rapt.Re
+    c = {"equal": np.ones(n), "spread": ((np.arange(n) + 1.0) / n) ** 2}[costs]
+    S[N.S_V] = 1e8 * c
+    S[N.S_DT] = 1.0
+    b = N.Batch(ctx, n)
+    b.upload(S, np.zeros(n, np.int32))
+    b.set_rows(5, np.full(n, 1, np.int64))
+    desc = N.make_desc(N.MODE_GC, rapt.params, 1.0)
+    for how in ("uploaded", "set_cost"):
+        if how == "set_cost":
+            b.set_cost(c)
+        b.run(desc)
+        assert kernel in rt.fake_last_kernel.value.decode(), rt.fake_last_kernel.value
+        assert rt.fake_last_grid.value * rt.fake_last_block.value == lanes
+
+
+_Q, _O, _MIX = "k_trace_gcnILi%dELi4E", "k_trace_gcnILi%dELi8E", "k_trace_gcmixILi%dE"
+ONE = 65536  # lanes of one wave a SIMD
+
+
+@pytest.mark.parametrize("name,model,n,costs,kernel,lanes", [
+    # particles that cost the same: none wait for others to end
+    ("double", 2, 8192, "equal", _O, ONE), ("double", 2, 8193, "equal", _Q, 4 * 8193 + 60),
+    ("double", 2, 16384, "equal", _Q, ONE), ("dipole", 1, 32768, "equal", _Q, 2 * ONE),
+    ("uniform", 8, 40000, "equal", _Q, 160000), ("double", 2, 65536, "equal", _MIX, 2 * ONE + 64),
+    # of different cost: one wave a SIMD, refilled
+    ("double", 2, 16384, "spread", _O, ONE), ("double", 2, 32768, "spread", _Q, ONE),
+    ("double", 2, 65536, "spread", _MIX, ONE), ("grid", 9, 16384, "equal", _O, ONE),
+    # fields that the order says nothing of, or with short steps
+    ("sheet", 7, 40000, "spread", _Q, 160000), ("sheet", 7, 131072, "spread", _Q, 8 * ONE),
+    ("bz", 3, 8192, "equal", _Q, 32768), ("bz", 3, 1, "equal", _Q, 64)])
+def test_default_guiding_centre_layout(fake, name, model, n, costs, kernel, lanes):
+    _run(fake, "case_layout", name, n, costs, kernel % model, lanes)
 
 
 if __name__ == "__main__":
