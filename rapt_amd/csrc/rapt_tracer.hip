@@ -230,8 +230,10 @@ __global__ void k_fill_u64(unsigned long long* p, int n) {
 template <int M, int K>
 static void launch_trace(rapt_ctx* c, const KArgs& A, int block, int64_t lanes) {
   const int64_t g = (lanes + block - 1) / block;
-  // (an interpreted user-written field's time is the interpreter's)
-  if constexpr (M != F_VAR_EARTH_DIPOLE && (K == KIND_GC || M != F_EXPR)) {
+  // Full orbits and adaptive runs in an interpreted user-written field spend
+  // their time in the interpreter, in a gridded one on memory, where the static
+  // kernel is no faster (a grid's 131,072 protons 6.4 ms, static 6.7; 1,024 1.87, 1.94)
+  if constexpr (M != F_VAR_EARTH_DIPOLE && (K == KIND_GC || (M != F_EXPR && M != F_GRID))) {
     if (trace_use_sp<M>(A)) {
       hipLaunchKernelGGL((k_trace<M, K, RAPT_PREC_FP64, true>), dim3((unsigned)g), dim3(block),
                          0, c->stream, A);
@@ -794,11 +796,15 @@ int rapt_batch_set_rows(rapt_batch* b, int32_t width, const int64_t* row_cap) {
 // is faster with its particles spread over more waves, up to one a SIMD
 // (current-sheet protons, spread so and packed: 100 3.7 and 7.9 ms, 500 4.3 and
 // 9.1, 4,096 7.5 and 9.6, 32,768 8.7 and 9.3; with two waves a SIMD 4,096 take
-// 8.1 and 32,768 11.3).
+// 8.1 and 32,768 11.3).  A gridded field waits for memory, and the waves of fewer
+// particles each ask for more of it: there only particles that get a wave of
+// their own are spread (256 on a grid of three times 7.4 and 9.1, 1,000 10.4
+// and 11.2; with several a wave 8,192 7.1 and 6.5, 16,384 7.2 and 6.7).
 // Full-orbit and guiding-centre runs take one path and are not: 4,096 protons
 // 6.3 ms packed and 7.6 spread, 1,000 guiding centres on octets 5.0 and 6.3.
 static constexpr int SPREAD_WAVES = 4;  // waves a CU: one a SIMD
-static int spread_lanes(int64_t n, int64_t waves) {
+static int spread_lanes(int64_t n, int64_t waves, bool grid) {
+  if (grid) return n <= waves ? 1 : 64;
   int wl = 64;
   while (wl > 1 && (n + wl / 2 - 1) / (wl / 2) <= waves) wl /= 2;
   return wl;
@@ -1013,7 +1019,8 @@ static int prepare_run(rapt_batch* b, const rapt_trace_desc* d, KArgs& A, int& b
   int block = d->block > 0 ? d->block : 0;
   A.wave_lanes = 64;
   if (d->mode == RAPT_MODE_ADAPTIVE && d->lanes <= 0) {
-    A.wave_lanes = spread_lanes(b->n, (int64_t)SPREAD_WAVES * cus);
+    A.wave_lanes = spread_lanes(b->n, (int64_t)SPREAD_WAVES * cus,
+                                c->field.model == RAPT_FIELD_GRID);
     lanes = (b->n + A.wave_lanes - 1) / A.wave_lanes * 64;
   }
   if (block == 0) {

@@ -141,6 +141,35 @@ def test_default_guiding_centre_layout(fake, name, model, n, costs, kernel, lane
     _run(fake, "case_layout", name, n, costs, kernel % model, lanes)
 
 
+# ---- full orbits and adaptive runs ---------------------------------------------------
+
+
+def case_orbits(rt, name, mode, n, kernel, waves):
+    ctx = _ctx(_field(name))
+    S = np.zeros((N.NSLOT, n))
+    S[N.S_Y0] = 5 * rapt.Re
+    b = N.Batch(ctx, n)
+    b.upload(S, np.zeros(n, np.int32))
+    b.set_rows(N.ROW_WIDTH[mode], np.full(n, 1, np.int64))
+    b.run(N.make_desc(mode, dict(rapt.params, GCtimestep=0.1), 1.0))
+    assert kernel in rt.fake_last_kernel.value.decode(), rt.fake_last_kernel.value
+    assert rt.fake_last_grid.value * rt.fake_last_block.value == 64 * waves
+
+
+_P, _A = N.MODE_PARTICLE, N.MODE_ADAPTIVE
+
+
+@pytest.mark.parametrize("name,mode,n,kernel,waves", [
+    # the static kernel where it is the faster one
+    ("dipole", _P, 1024, "ILi1ELi0ELi0ELb1E", 16), ("grid", _P, 1024, "ILi9ELi0ELi0ELb0E", 16),
+    ("dipole", _A, 4096, "ILi1ELi2ELi0ELb1E", 1024), ("user", _P, 64, "ILi10ELi0ELi0ELb0E", 1),
+    # on a grid, a wave each or 64 a wave
+    ("grid", _A, 1, "ILi9ELi2ELi0ELb0E", 1), ("grid", _A, 1024, "ILi9ELi2ELi0ELb0E", 1024),
+    ("grid", _A, 1025, "ILi9ELi2ELi0ELb0E", 17), ("grid", _A, 16384, "ILi9ELi2ELi0ELb0E", 256)])
+def test_orbit_kernels_and_spread(fake, name, mode, n, kernel, waves):
+    _run(fake, "case_orbits", name, mode, n, kernel, waves)
+
+
 if __name__ == "__main__":
     _lib = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
     globals()[sys.argv[2]](_Var(_lib), *[int(a) if a.lstrip("-").isdigit() else a
