@@ -156,6 +156,11 @@ typedef struct rapt_batch rapt_batch;
 /* ---- context ---------------------------------------------------------- */
 int rapt_ctx_create(int device, rapt_ctx **out);
 int rapt_ctx_destroy(rapt_ctx *ctx);
+/* A context keeps up to 2.5 GiB of device scratch between the calls that take
+ * and return host arrays.  Its own allocations take it back when memory runs
+ * out; this frees it for other users of the device (the next such call
+ * allocates again). */
+int rapt_ctx_release_scratch(rapt_ctx *ctx);
 const char *rapt_last_error(rapt_ctx *ctx);
 /* replaces the field object handed to the tracer constructors */
 int rapt_field_set(rapt_ctx *ctx, const rapt_field_desc *field);

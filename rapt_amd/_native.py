@@ -83,6 +83,7 @@ def lib():
         C.POINTER(C.c_int64)
     L.rapt_ctx_create.argtypes = [C.c_int, C.POINTER(vp)]
     L.rapt_ctx_destroy.argtypes = [vp]
+    L.rapt_ctx_release_scratch.argtypes = [vp]
     L.rapt_last_error.argtypes = [vp]
     L.rapt_last_error.restype = C.c_char_p
     L.rapt_field_set.argtypes = [vp, C.POINTER(FieldDesc)]
@@ -135,7 +136,8 @@ def lib():
     # device pointers (as integers) for the allocation-free entry point
     L.rapt_trace_device_noalloc.argtypes = [vp, C.POINTER(TraceDesc), C.c_int64, vp, vp, vp,
                                             vp, vp, vp, vp, vp, vp, C.POINTER(Counters)]
-    for nm in ("rapt_ctx_create", "rapt_ctx_destroy", "rapt_field_set", "rapt_field_eval",
+    for nm in ("rapt_ctx_create", "rapt_ctx_destroy", "rapt_ctx_release_scratch",
+               "rapt_field_set", "rapt_field_eval",
                "rapt_halfbounce", "rapt_bounce_labels", "rapt_bounce_center_advance",
                "rapt_bounce_center_equatorial",
                "rapt_batch_epochs_begin", "rapt_batch_epoch_next", "rapt_batch_epochs_end",
@@ -184,6 +186,11 @@ class Context:
         if rc != 0:
             msg = lib().rapt_last_error(self.h)
             raise RuntimeError("%s failed (%d): %s" % (what, rc, msg.decode() if msg else ""))
+
+    def release_scratch(self):
+        """Frees the device scratch (up to 2.5 GiB) that the context keeps
+        between calls, for other users of the device."""
+        self.check(lib().rapt_ctx_release_scratch(self.h), "rapt_ctx_release_scratch")
 
     def set_field(self, desc):
         grid = desc.get("grid")

@@ -373,13 +373,13 @@ extern "C" int rapt_bounce_center_equatorial(rapt_ctx* c, int64_t n, double* tpo
   int64_t *d_nrow = nullptr, *d_off = nullptr, *d_acc = nullptr;
   int32_t* d_st = nullptr;
   int rc = RAPT_OK;
-  if (hipMalloc(&d_tpos, sizeof(double) * 4 * n) != hipSuccess ||
-      hipMalloc(&d_in, sizeof(double) * 6 * n) != hipSuccess ||
-      hipMalloc(&d_rows, sizeof(double) * 4 * (total > 0 ? total : 1)) != hipSuccess ||
-      hipMalloc(&d_nrow, sizeof(int64_t) * n) != hipSuccess ||
-      hipMalloc(&d_off, sizeof(int64_t) * n) != hipSuccess ||
-      hipMalloc(&d_acc, sizeof(int64_t) * n) != hipSuccess ||
-      hipMalloc(&d_st, sizeof(int32_t) * n) != hipSuccess) {
+  if (ctx_malloc(c, &d_tpos, sizeof(double) * 4 * n) != hipSuccess ||
+      ctx_malloc(c, &d_in, sizeof(double) * 6 * n) != hipSuccess ||
+      ctx_malloc(c, &d_rows, sizeof(double) * 4 * (total > 0 ? total : 1)) != hipSuccess ||
+      ctx_malloc(c, &d_nrow, sizeof(int64_t) * n) != hipSuccess ||
+      ctx_malloc(c, &d_off, sizeof(int64_t) * n) != hipSuccess ||
+      ctx_malloc(c, &d_acc, sizeof(int64_t) * n) != hipSuccess ||
+      ctx_malloc(c, &d_st, sizeof(int32_t) * n) != hipSuccess) {
     rc = set_err(c, RAPT_E_OOM, "BounceCenter allocation failed");
   } else {
     BCArgs C;

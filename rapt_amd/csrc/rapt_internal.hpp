@@ -124,8 +124,10 @@ struct Workspace {
     c->ws_bytes = 0;
   }
 };
-// hipMalloc that takes back the kept scratch when memory runs out
-static inline hipError_t ctx_malloc(rapt_ctx* c, void** p, size_t bytes) {
+// hipMalloc that takes back the kept scratch when memory runs out: for every
+// allocation of a context beside its scratch (not while a Workspace is held)
+template <class T>
+static inline hipError_t ctx_malloc(rapt_ctx* c, T** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e != hipSuccess) {
     (void)hipGetLastError();

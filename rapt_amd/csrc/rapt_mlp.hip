@@ -784,11 +784,11 @@ static int mlp_work(rapt_mlp* m, int bt) {
   mlp_free_work(m);
   rapt_ctx* c = m->ctx;
   const size_t act = (size_t)m->members * 2 * bt * H;
-  bool ok = hipMalloc(&m->X, sizeof(float) * 3 * bt) == hipSuccess &&
-            hipMalloc(&m->Y, sizeof(float) * 3 * bt * m->members) == hipSuccess &&
-            hipMalloc(&m->hp, sizeof(bf16) * act) == hipSuccess &&
-            hipMalloc(&m->zp, sizeof(bf16) * act) == hipSuccess &&
-            hipMalloc(&m->part, sizeof(float) * m->members * (bt / TB) * NSLOT_G * H) ==
+  bool ok = ctx_malloc(c, &m->X, sizeof(float) * 3 * bt) == hipSuccess &&
+            ctx_malloc(c, &m->Y, sizeof(float) * 3 * bt * m->members) == hipSuccess &&
+            ctx_malloc(c, &m->hp, sizeof(bf16) * act) == hipSuccess &&
+            ctx_malloc(c, &m->zp, sizeof(bf16) * act) == hipSuccess &&
+            ctx_malloc(c, &m->part, sizeof(float) * m->members * (bt / TB) * NSLOT_G * H) ==
                 hipSuccess;
   if (!ok) {
     mlp_free_work(m);
@@ -897,17 +897,17 @@ int rapt_mlp_create(rapt_ctx* c, int32_t members, const float* theta0, double ma
   m->mass = mass;
   m->eV = eV;
   const size_t np = (size_t)members * NPAD;
-  bool ok = hipMalloc(&m->theta, sizeof(float) * np) == hipSuccess &&
-            hipMalloc(&m->grad, sizeof(float) * np) == hipSuccess &&
-            hipMalloc(&m->m1, sizeof(float) * np) == hipSuccess &&
-            hipMalloc(&m->m2, sizeof(float) * np) == hipSuccess &&
-            hipMalloc(&m->wb, sizeof(bf16) * np) == hipSuccess &&
-            hipMalloc(&m->packed, sizeof(bf16) * members * 2 * PACKED) == hipSuccess &&
-            hipMalloc(&m->p1, sizeof(bf16) * members * P1SIZE) == hipSuccess &&
-            hipMalloc(&m->fw, sizeof(bf16) * members * 2 * PACKED) == hipSuccess &&
-            hipMalloc(&m->bw, sizeof(bf16) * members * 2 * PACKED) == hipSuccess &&
-            hipMalloc(&m->loss, sizeof(double) * members) == hipSuccess &&
-            hipMalloc(&m->norm, sizeof(float) * 6) == hipSuccess;
+  bool ok = ctx_malloc(c, &m->theta, sizeof(float) * np) == hipSuccess &&
+            ctx_malloc(c, &m->grad, sizeof(float) * np) == hipSuccess &&
+            ctx_malloc(c, &m->m1, sizeof(float) * np) == hipSuccess &&
+            ctx_malloc(c, &m->m2, sizeof(float) * np) == hipSuccess &&
+            ctx_malloc(c, &m->wb, sizeof(bf16) * np) == hipSuccess &&
+            ctx_malloc(c, &m->packed, sizeof(bf16) * members * 2 * PACKED) == hipSuccess &&
+            ctx_malloc(c, &m->p1, sizeof(bf16) * members * P1SIZE) == hipSuccess &&
+            ctx_malloc(c, &m->fw, sizeof(bf16) * members * 2 * PACKED) == hipSuccess &&
+            ctx_malloc(c, &m->bw, sizeof(bf16) * members * 2 * PACKED) == hipSuccess &&
+            ctx_malloc(c, &m->loss, sizeof(double) * members) == hipSuccess &&
+            ctx_malloc(c, &m->norm, sizeof(float) * 6) == hipSuccess;
   if (!ok) {
     rapt_mlp_destroy(m);
     return set_err(c, RAPT_E_OOM, "MLP allocation failed");
@@ -992,10 +992,10 @@ int rapt_mlp_targets(rapt_mlp* m, int64_t n, const float* query, const double* l
   float *dq = nullptr, *dX = nullptr, *dT = nullptr;
   double* dl = nullptr;
   int rc = RAPT_OK;
-  if (hipMalloc(&dq, sizeof(float) * 3 * n) != hipSuccess ||
-      hipMalloc(&dl, sizeof(double) * 3 * n) != hipSuccess ||
-      hipMalloc(&dX, sizeof(float) * 3 * n) != hipSuccess ||
-      hipMalloc(&dT, sizeof(float) * 3 * n) != hipSuccess) {
+  if (ctx_malloc(c, &dq, sizeof(float) * 3 * n) != hipSuccess ||
+      ctx_malloc(c, &dl, sizeof(double) * 3 * n) != hipSuccess ||
+      ctx_malloc(c, &dX, sizeof(float) * 3 * n) != hipSuccess ||
+      ctx_malloc(c, &dT, sizeof(float) * 3 * n) != hipSuccess) {
     rc = set_err(c, RAPT_E_OOM, "targets allocation failed");
   } else if (hipMemcpyAsync(dq, query, sizeof(float) * 3 * n, hipMemcpyHostToDevice,
                             c->stream) != hipSuccess ||

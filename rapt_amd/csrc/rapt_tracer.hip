@@ -297,6 +297,13 @@ int rapt_ctx_create(int device, rapt_ctx** out) {
   return RAPT_OK;
 }
 
+int rapt_ctx_release_scratch(rapt_ctx* c) {
+  if (!c) return RAPT_E_ARG;
+  HIP_OK(c, hipSetDevice(c->device));
+  Workspace(c).drop();
+  return RAPT_OK;
+}
+
 int rapt_ctx_destroy(rapt_ctx* c) {
   if (!c) return RAPT_E_ARG;
   (void)hipSetDevice(c->device);
@@ -373,7 +380,7 @@ int rapt_field_expr_set(rapt_ctx* c, int32_t nb, int32_t ne, const int32_t* code
   const size_t kb = sizeof(double) * (size_t)(nconst > 0 ? nconst : 1);
   const size_t cb = sizeof(int32_t) * 4 * (size_t)(nb + ne);
   void* mem = nullptr;
-  if (hipMalloc(&mem, kb + cb) != hipSuccess)
+  if (ctx_malloc(c, &mem, kb + cb) != hipSuccess)
     return set_err(c, RAPT_E_OOM, "field program allocation failed");
   if ((nconst > 0 && hipMemcpy(mem, consts, sizeof(double) * nconst, hipMemcpyHostToDevice) !=
                          hipSuccess) ||
@@ -427,7 +434,7 @@ int rapt_grid_set(rapt_ctx* c, int32_t nx, int32_t ny, int32_t nz, int32_t nt, c
     }
   }
   double* mem = nullptr;
-  if (ctx_malloc(c, (void**)&mem, sizeof(double) * total) != hipSuccess)
+  if (ctx_malloc(c, &mem, sizeof(double) * total) != hipSuccess)
     return set_err(c, RAPT_E_OOM, "grid allocation of %zu bytes failed", sizeof(double) * total);
   if (hipMemcpy(mem, h.data(), sizeof(double) * total, hipMemcpyHostToDevice) != hipSuccess) {
     (void)hipFree(mem);
@@ -441,11 +448,15 @@ int rapt_grid_set(rapt_ctx* c, int32_t nx, int32_t ny, int32_t nz, int32_t nt, c
   const size_t cell_bytes = sizeof(double) * 32 * ncell * (E ? 2 : 1);
   size_t free_b = 0, total_b = 0;
   (void)hipMemGetInfo(&free_b, &total_b);
+  if (cell_bytes > free_b / 2) {  // the kept scratch counts as free
+    Workspace(c).drop();
+    (void)hipMemGetInfo(&free_b, &total_b);
+  }
   double* cells = nullptr;
   const char* pts = getenv("RAPT_GRID_POINTS");  // "1": keep the point layout
   const bool want_cells = !(pts && pts[0] == '1');
   if (want_cells && cell_bytes <= ((size_t)64 << 30) && cell_bytes <= free_b / 2 &&
-      hipMalloc(&cells, cell_bytes) == hipSuccess) {
+      ctx_malloc(c, &cells, cell_bytes) == hipSuccess) {
     const int64_t nthr = (int64_t)ncell * 8;
     const unsigned nblk = (unsigned)((nthr + 255) / 256);
     hipLaunchKernelGGL(k_grid_cells, dim3(nblk), dim3(256), 0, c->stream, mem + offB, cells,
@@ -510,7 +521,7 @@ int rapt_rhs_eval(rapt_ctx* c, int32_t mode, int32_t eom, int32_t enforce_equato
             wo = mode == RAPT_MODE_PARTICLE ? 6 : 4;
   HIP_OK(c, hipSetDevice(c->device));
   double* mem = nullptr;
-  if (hipMalloc(&mem, sizeof(double) * (size_t)(wi + wk + wo) * n) != hipSuccess)
+  if (ctx_malloc(c, &mem, sizeof(double) * (size_t)(wi + wk + wo) * n) != hipSuccess)
     return set_err(c, RAPT_E_OOM, "rhs: allocation failed");
   double *dty = mem, *dk = mem + (size_t)wi * n, *dout = mem + (size_t)(wi + wk) * n;
   int rc = RAPT_OK;
@@ -638,7 +649,7 @@ int rapt_batch_create(rapt_ctx* c, int64_t n, rapt_batch** out) {
   };
   parts();
   const size_t bytes = (size_t)at;
-  if (ctx_malloc(c, (void**)&b->mem, bytes) != hipSuccess) {
+  if (ctx_malloc(c, &b->mem, bytes) != hipSuccess) {
     b->mem = nullptr;
     rapt_batch_destroy(b);
     return set_err(c, RAPT_E_OOM, "device allocation of a %lld-particle batch failed",
@@ -768,7 +779,7 @@ int rapt_batch_set_rows(rapt_batch* b, int32_t width, const int64_t* row_cap) {
     (void)hipFree(b->d_rows);
     b->d_rows = nullptr;
     if (tot > 0 &&
-        ctx_malloc(c, (void**)&b->d_rows, sizeof(double) * width * tot) != hipSuccess) {
+        ctx_malloc(c, &b->d_rows, sizeof(double) * width * tot) != hipSuccess) {
       free(off);
       b->total_rows = 0;
       return set_err(c, RAPT_E_OOM, "trajectory buffer of %lld rows failed", (long long)tot);
@@ -1288,10 +1299,10 @@ int rapt_batch_epochs_begin(rapt_batch* b, const rapt_trace_desc* desc,
   HIP_OK(c, hipSetDevice(c->device));
   const int64_t n = b->n;
   const size_t nr = (size_t)n * rows_per_epoch;
-  bool ok = ctx_malloc(c, (void**)&b->d_erows, sizeof(double) * nr * width) == hipSuccess &&
-            hipMalloc(&b->d_eoff, sizeof(int64_t) * n) == hipSuccess &&
-            hipMalloc(&b->d_ecap, sizeof(int64_t) * n) == hipSuccess &&
-            hipMalloc(&b->d_left, sizeof(int32_t)) == hipSuccess &&
+  bool ok = ctx_malloc(c, &b->d_erows, sizeof(double) * nr * width) == hipSuccess &&
+            ctx_malloc(c, &b->d_eoff, sizeof(int64_t) * n) == hipSuccess &&
+            ctx_malloc(c, &b->d_ecap, sizeof(int64_t) * n) == hipSuccess &&
+            ctx_malloc(c, &b->d_left, sizeof(int32_t)) == hipSuccess &&
             hipHostMalloc(&b->h_rows, sizeof(double) * nr * width, 0) == hipSuccess &&
             hipHostMalloc(&b->h_nrows, sizeof(int64_t) * n, 0) == hipSuccess &&
             hipHostMalloc(&b->h_status, sizeof(int32_t) * n, 0) == hipSuccess &&

@@ -170,6 +170,90 @@ def test_orbit_kernels_and_spread(fake, name, mode, n, kernel, waves):
     _run(fake, "case_orbits", name, mode, n, kernel, waves)
 
 
+# ---- kept scratch --------------------------------------------------------------------
+
+
+def _keep_scratch(rt, ctx):
+    """A call that leaves the context with scratch; what is free beside it."""
+    f = _field("dipole")
+    n = 65536
+    tpos = np.tile([0.0, 5 * rapt.Re, 0.0, 0.0], (n, 1))
+    ctx.halfbounce(f.descriptor(), tpos, np.full(n, 1e-5), 50)
+    assert rt.fake_used.value > 2 * GIB
+
+
+def case_memory(rt, call):
+    """Every allocation that the call makes beside the kept scratch: with that
+    much free and less, where the scratch has to give."""
+    dip = _field("dipole")
+    ctx = _ctx(dip)
+    tp = np.array([[0.0, 5 * rapt.Re, 0.0, 0.0]])
+    net = None
+    if call in ("train", "forward", "targets"):
+        from rapt_amd import surrogate as SG
+        net = SG.Surrogate(dip, members=2)
+    b = N.Batch(ctx, 1000) if call in ("epochs", "set_rows") else None
+    if call == "epochs":
+        b.upload(np.ones((N.NSLOT, 1000)), np.zeros(1000, np.int32))
+        b.set_rows(7, np.ones(1000, np.int64))
+
+    def run():
+        if call == "train":
+            z = np.zeros((4096, 3), np.float32)
+            net.train_steps(z, z, np.zeros(4096, np.int64), 4096, 1e-3, 1e-3)
+        elif call == "forward":
+            net.forward(np.zeros((4096, 3), np.float32))
+        elif call == "targets":
+            net.targets(np.ones((4096, 3)), np.ones((4096, 3)))
+        elif call == "surrogate":
+            from rapt_amd import surrogate as SG
+            SG.Surrogate(dip, members=2).close()
+        elif call == "equatorial":
+            ctx.bounce_center_equatorial(dip.descriptor(), np.tile(tp, (999, 1)), 1.0, 1.0, 0.0,
+                                         3, 1e-6, 1e-6)
+        elif call == "epochs":
+            for _ in b.epochs(N.make_desc(N.MODE_PARTICLE, rapt.params, 1.0), 4, 1):
+                pass
+        elif call == "rhs":
+            ctx.rhs_eval(dip.descriptor(), N.MODE_GC, np.ones((999, 5)), np.ones((999, 4)))
+        elif call == "program":
+            ctx.set_field(_field("user").descriptor())
+        elif call == "grid":
+            ctx.set_field(_Grid(["0"]).descriptor())
+            assert b"k_grid_cells" in rt.fake_last_kernel.value  # (the faster layout)
+        elif call == "batch":
+            N.Batch(ctx, 1000).close()
+        else:
+            b.set_rows(7, np.full(1000, 10, np.int64))
+
+    for room in (0, 64, 4096, 100000, 1 << 20, 3 << 20):
+        ctx.set_field(dip.descriptor())
+        rt.fake_budget.value = 1 << 40
+        _keep_scratch(rt, ctx)
+        rt.fake_budget.value = rt.fake_used.value + room
+        run()
+
+
+@pytest.mark.parametrize("call", ["train", "forward", "targets", "surrogate", "equatorial",
+                                  "epochs", "rhs", "program", "grid", "batch", "set_rows"])
+def test_kept_scratch_is_given_back_to_calls(fake, call):
+    _run(fake, "case_memory", call)
+
+
+def case_release(rt):
+    ctx = _ctx(_field("dipole"))
+    before = rt.fake_used.value
+    _keep_scratch(rt, ctx)
+    ctx.release_scratch()
+    assert rt.fake_used.value == before
+    ctx.release_scratch()
+    _keep_scratch(rt, ctx)
+
+
+def test_kept_scratch_is_given_back_on_request(fake):
+    _run(fake, "case_release")
+
+
 if __name__ == "__main__":
     _lib = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
     globals()[sys.argv[2]](_Var(_lib), *[int(a) if a.lstrip("-").isdigit() else a
