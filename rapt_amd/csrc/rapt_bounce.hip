@@ -176,6 +176,7 @@ static int run_bounce(rapt_ctx* c, int64_t n, const double* in, int in_w, const 
             hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
       return set_err(c, RAPT_E_HIP, "bounce kernel failed");
+    ws.done();
     if (cap == CAP_MOST || !any_overflow(status, n)) return RAPT_OK;
   }
 }
@@ -335,6 +336,7 @@ extern "C" int rapt_bounce_center_advance(rapt_ctx* c, int64_t n, double* tpos, 
             hipSuccess ||
         hipStreamSynchronize(c->stream) != hipSuccess)
       return set_err(c, RAPT_E_HIP, "BounceCenter results failed to copy");
+    ws.done();
     return RAPT_OK;
   }
 }

@@ -82,6 +82,7 @@ extern "C" int rapt_particle_gc(rapt_ctx* c, int64_t n, const double* rows, cons
              hipSuccess ||
          hipStreamSynchronize(c->stream) != hipSuccess))
       rc = set_err(c, RAPT_E_HIP, "diagnostics kernel failed");
+    if (rc == RAPT_OK) ws.done();
   }
   return rc;
 }

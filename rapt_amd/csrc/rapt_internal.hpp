@@ -95,16 +95,20 @@ static inline int set_err(rapt_ctx* c, int code, const char* fmt, ...) {
 // The context's device scratch for the length of one entry point's call: held
 // under a lock, so calls from several threads take turns, grown when a call
 // needs more, and kept for the next call up to KEEP bytes (allocating and
-// freeing 2 GiB costs about 2 ms a call).  A call ends with its stream
-// synchronised, so nothing reads the scratch once the lock is dropped.
+// freeing 2 GiB costs about 2 ms a call).  A call that ends well has synchronised
+// its stream and says so (done); one that fails half way has it done here.
+// Nothing uses the scratch, or the caller's arrays, once the lock is dropped.
 struct Workspace {
   static constexpr size_t KEEP = (size_t)5 << 29;  // 2.5 GiB
   rapt_ctx* c;
+  bool queued = false;  // there may be work on the stream that uses the scratch
   std::lock_guard<std::mutex> lock;
   explicit Workspace(rapt_ctx* ctx) : c(ctx), lock(ctx->ws_mu) {}
   ~Workspace() {
+    if (queued) (void)hipStreamSynchronize(c->stream);
     if (c->ws_bytes > KEEP) drop();
   }
+  void done() { queued = false; }
   // at least `bytes` bytes, or nullptr; what an earlier get returned is void
   char* get(size_t bytes) {
     if (c->ws_bytes < bytes) {
@@ -116,6 +120,7 @@ struct Workspace {
       }
       c->ws_bytes = bytes;
     }
+    queued = true;
     return static_cast<char*>(c->ws);
   }
   void drop() {

@@ -875,6 +875,7 @@ static int infer(rapt_mlp* m, int64_t n, const float* query, float thresh, float
       (raw && rapt_copy_out(c, raw, draw, sizeof(float) * nraw) != hipSuccess) ||
       hipStreamSynchronize(st) != hipSuccess)
     return set_err(c, RAPT_E_HIP, "inference kernel failed");
+  ws.done();
   if (kernel_ms) {
     float ms = 0.0f;
     (void)hipEventElapsedTime(&ms, c->ev0, c->ev1);
@@ -1091,6 +1092,7 @@ int rapt_mlp_train(rapt_mlp* m, int64_t n, const float* X, const float* T, int32
   }
   if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
     rc = rc ? rc : set_err(c, RAPT_E_HIP, "training kernels failed");
+  if (rc == RAPT_OK) ws.done();
   m->packed_ok = false;
   return rc;
 }

@@ -616,6 +616,8 @@ int rapt_field_eval(rapt_ctx* c, int what, int64_t n, const double* tpos, double
                (rapt_copy_out(c, out, dout, sizeof(double) * w * n) != hipSuccess ||
                 hipStreamSynchronize(c->stream) != hipSuccess)) {
       rc = set_err(c, RAPT_E_HIP, "field eval failed");
+    } else if (rc == RAPT_OK) {
+      ws.done();
     }
   }
   return rc;

@@ -254,6 +254,46 @@ def test_kept_scratch_is_given_back_on_request(fake):
     _run(fake, "case_release")
 
 
+# ---- calls that fail half way ----------------------------------------------------------
+
+
+def case_failed_copy(rt, call):
+    """The k-th copy fails, for every k that the call reaches: it raises, and
+    leaves nothing on the stream that could still use its arrays."""
+    from rapt_amd import surrogate as SG
+    dip = _field("dipole")
+    ctx, d = _ctx(dip), dip.descriptor()
+    n = 700000 if call in ("field_eval", "particle_gc") else 50  # (staged copies: 4 MB)
+    tp = np.tile([0.0, 5 * rapt.Re, 0.0, 0.0], (n, 1))
+    net = SG.Surrogate(dip, members=2) if call in ("train", "infer", "values") else None
+    q = np.ones((1 << 18 if call == "values" else 50, 3), np.float32)
+    fn = {"halfbounce": lambda: ctx.halfbounce(d, tp, 1e-5, 50),
+          "labels": lambda: ctx.bounce_labels(d, np.ones((n, 3)), 1.0, 1.0, 1e3, 50),
+          "centres": lambda: ctx.bounce_center_advance(d, tp, 1e-5, 1.0, 1.0, 0.0, 2, 1e-6, 1e-6,
+                                                       1e3, 50),
+          "field_eval": lambda: ctx.field_eval(d, "B", tp),
+          "particle_gc": lambda: ctx.particle_gc(d, np.ones((n, 7)), 1.0, 1.0),
+          "infer": lambda: net.infer(q, raw=True), "values": lambda: net.infer(q, raw=True),
+          "train": lambda: net.train_steps(q[:50], q[:50], np.zeros(64, np.int64), 64, 1e-3, 1e-3,
+                                           want_grad=True)}[call]
+    for k in range(100):
+        rt.fake_fail_copy.value = k
+        try:
+            fn()
+        except RuntimeError:
+            assert rt.fake_pending.value == 0, k
+            rt._lib.hipGetLastError()
+        else:
+            break
+    assert 1 < k < 99
+
+
+@pytest.mark.parametrize("call", ["halfbounce", "labels", "centres", "field_eval", "particle_gc",
+                                  "infer", "values", "train"])
+def test_failed_calls_leave_nothing_queued(fake, call):
+    _run(fake, "case_failed_copy", call)
+
+
 if __name__ == "__main__":
     _lib = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
     globals()[sys.argv[2]](_Var(_lib), *[int(a) if a.lstrip("-").isdigit() else a
