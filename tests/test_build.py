@@ -21,7 +21,7 @@ def built(tmp_path):
     obj.mkdir(parents=True)
     for path in [p for p in tmp_path.rglob("*") if p.is_file()]:
         os.utime(path, (1e9, 1e9))
-    for k, name in enumerate(["rapt_jit_headers.inc"] + [o + s for s in (".d", ".o")
+    for k, name in enumerate(["rapt_jit_headers.inc"] + [o + s for s in (".o", ".d")
                                                          for o in OBJECTS]):
         dep = "rapt_gcn_kernel.hpp" if name == "rapt_gcn.d" else ""
         (obj / name).write_text("%s: %s\n" % ("../lib/obj/rapt_gcn.o", dep) if dep else "")
