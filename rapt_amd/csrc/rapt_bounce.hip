@@ -28,8 +28,8 @@ static void launch_lab(rapt_ctx* c, const BounceArgs& A, const LabelArgs& L, uns
 
 // From ORDER_MIN queries on a batch's lines are taken in k_line_order's order
 // (65,536 lines: 1.24 -> 0.82 ms, 16,384 labels with every wave resident
-// 1.5 -> 1.25, its own launch 10 us); below, the longest line's own time is the launch's and order changes
-// nothing.
+// 1.5 -> 1.25, its own launch 10 us); below, the longest line's own time is the
+// launch's and order changes nothing.
 static constexpr int64_t ORDER_MIN = 4096;
 template <int M>
 static void launch_order(rapt_ctx* c, const BounceArgs& A, bool labels, int32_t* order) {
@@ -43,6 +43,12 @@ static void launch_order(rapt_ctx* c, const BounceArgs& A, bool labels, int32_t*
 // two waves a SIMD for 2 GiB of scratch.  Only when a line overflows it is
 // the call repeated with CAP_MOST and 16,384 lines in the same memory.
 static constexpr int32_t CAP_FIRST = 512, CAP_MOST = 2048;
+static constexpr int64_t WAVES_FIRST = 2048;  // resident, at CAP_FIRST points
+static constexpr int64_t resident_waves(int32_t cap) { return WAVES_FIRST * CAP_FIRST / cap; }
+// (pt addresses the points by 32-bit offsets)
+static_assert((uint64_t)resident_waves(CAP_FIRST) * wave_bytes(CAP_FIRST) <= UINT32_MAX &&
+              (uint64_t)resident_waves(CAP_MOST) * wave_bytes(CAP_MOST) <= UINT32_MAX,
+              "the points' scratch has 32-bit offsets");
 
 // Waves of a surrogate-label launch in a dipole-type field.  No resource asks
 // for this limit: with every wave resident 65,536 queries take 5.2 ms and
@@ -64,14 +70,14 @@ static constexpr int64_t LABEL_WAVES = 72;
 // not fit.
 static unsigned bounce_scratch(Workspace& ws, BounceArgs& A, int64_t n, int32_t cap, bool groups,
                                bool positions, int64_t waves, size_t extra, char** extra_mem) {
-  int64_t most = (int64_t)2048 * CAP_FIRST / cap;  // resident waves
+  int64_t most = resident_waves(cap);
   if (waves > 0 && most > waves) most = waves;
   const int64_t per_wave = groups ? GRP_PER_WAVE : 32;
   int64_t blocks = (n + per_wave - 1) / per_wave;
   if (blocks > most) blocks = most;
   A.cap = cap;
   A.slots = n < blocks * per_wave ? n : blocks * per_wave;
-  const size_t pts = (size_t)blocks * wave_bytes(cap);  // (32-bit offsets)
+  const size_t pts = (size_t)blocks * wave_bytes(cap);
   const size_t nz = positions ? (size_t)2 * cap * A.slots : 0;
   extra = (extra + 1023) / 1024 * 1024;
   char* mem = ws.get(extra + pts + sizeof(double) * 2 * nz);

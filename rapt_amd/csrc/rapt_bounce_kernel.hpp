@@ -44,8 +44,9 @@
 // Against one lane a line, with a binary search through the scratch, a cosine
 // and a sine at each of the 512 nodes, a |B| evaluation beside each point's
 // direction and 16,384 lanes at most: S_b of 65,536 lines 12.1 -> 0.80 ms,
-// labels 17.0 -> 1.2 ms (16,384 queries; 10.1 on the 72 waves they are launched
-// with, rapt_bounce.hip) and 14.8 -> 0.46 ms (300), five bounce centres over four
+// labels 17.0 -> 1.2 ms (16,384 queries with every wave; 9.9 on the 72 waves that
+// dipole-type fields' are launched with, rapt_bounce.hip) and 14.8 -> 0.46 ms
+// (300), five bounce centres over four
 // rows 400 -> 11.1 ms, the same results bit for bit.
 #pragma once
 #ifndef __HIPCC_RTC__
@@ -214,8 +215,9 @@ __device__ __forceinline__ double pair_swap(double v) {
   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
 }
 
-// The scratch value at a byte offset (at most 2 GiB): the address stays in
-// scalar registers and the offset is one 32-bit register.
+// The scratch value at a byte offset (unsigned: it reaches 2.01 GiB, and
+// rapt_bounce.hip holds it below 4): the address stays in scalar registers and
+// the offset is one 32-bit register.
 __device__ __forceinline__ double& pt(const BounceArgs& A, uint32_t off) {
   return *(double*)(A.pts + off);
 }
