@@ -42,8 +42,19 @@ void rapt_ring_free(rapt_ctx* c) {
   }
 }
 
+// Memory that the runtime knows (pinned, managed or a device's) takes the copy
+// as it is: PINNED.
+static bool known_to_runtime(const void* p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type != hipMemoryTypeUnregistered;
+}
+
 hipError_t rapt_copy_out(rapt_ctx* c, void* dst, const void* src, size_t bytes) {
-  if (bytes < COPY_MIN)
+  if (bytes < COPY_MIN || known_to_runtime(dst))
     return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream);
   std::lock_guard<std::mutex> lock(c->ring_mu);  // one copy at a time has the ring
   if (!ring_make(c)) {

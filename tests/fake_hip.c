@@ -22,7 +22,7 @@ size_t fake_overflow_bytes; /* the next copy from the device of this many bytes 
                                "too many points" (-20), then the option is off */
 int fake_pinned_lookup;    /* 1: every host pointer is one of the runtime's */
 int fake_copies;           /* asynchronous copies */
-size_t fake_largest_copy;  /* bytes */
+size_t fake_largest_copy;  /* bytes, of those from the device */
 const char* fake_last_kernel = "";
 unsigned fake_last_grid, fake_last_block;
 static hipError_t last;
@@ -79,7 +79,7 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hip
   if (fake_fail_copy > 0) --fake_fail_copy;
   ++fake_pending;
   ++fake_copies;
-  if (n > fake_largest_copy) fake_largest_copy = n;
+  if (k == hipMemcpyDeviceToHost && n > fake_largest_copy) fake_largest_copy = n;
   memcpy(d, s, n);
   if (k == hipMemcpyDeviceToHost && n && n == fake_overflow_bytes) {
     for (size_t i = 0; i < n / 4; ++i) ((int*)d)[i] = -20;

@@ -1,6 +1,7 @@
 """Results large enough for the staged copies (rapt_copy.hip), a megabyte a
 slot of a ring of eight: one slot short of the threshold, at it, a last slot
 that is not full, the ring more than once round; and from two threads at once."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -66,3 +67,21 @@ def test_inference_values_on_either_side_of_the_device_widening():
         np.testing.assert_array_equal(v, np.r_[a[0], b[0]])
         np.testing.assert_array_equal(flag, np.r_[a[1], b[1]])
         np.testing.assert_array_equal(raw, np.concatenate([a[2], b[2]], axis=1))
+
+
+def test_large_results_to_pinned_memory():
+    """A destination that the runtime has pinned takes the copy directly."""
+    f = F.EarthDipole().descriptor()
+    ctx = N.context()
+    tp = np.ascontiguousarray(_points(900003))
+    ref = ctx.field_eval(f, "B", tp)
+    hip = C.CDLL("libamdhip64.so")
+    p = C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(p), C.c_size_t(ref.nbytes), 0) == 0
+    try:
+        ptr = C.cast(p, C.POINTER(C.c_double))
+        ctx.check(N.lib().rapt_field_eval(ctx.h, N.EVAL["B"], len(tp), N._dp(tp), ptr),
+                  "rapt_field_eval")
+        np.testing.assert_array_equal(np.ctypeslib.as_array(ptr, ref.shape), ref)
+    finally:
+        hip.hipHostFree(p)

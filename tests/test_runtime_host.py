@@ -294,6 +294,25 @@ def test_failed_calls_leave_nothing_queued(fake, call):
     _run(fake, "case_failed_copy", call)
 
 
+# ---- large results ---------------------------------------------------------------------
+
+
+def case_destination(rt, known):
+    n = 700000
+    dip = _field("dipole")
+    ctx = _ctx(dip)
+    rt.fake_pinned_lookup.value = known
+    out = ctx.field_eval(dip.descriptor(), "magB", np.ones((n, 4)))
+    assert out.nbytes > 4 << 20
+    assert rt.fake_largest_copy.value == (out.nbytes if known else 1 << 20)
+    assert rt._lib.hipGetLastError() == 0  # (the runtime's "not mine" is no error of the call)
+
+
+@pytest.mark.parametrize("known", [0, 1])
+def test_large_results_to_the_runtimes_own_memory_are_one_copy(fake, known):
+    _run(fake, "case_destination", known)
+
+
 if __name__ == "__main__":
     _lib = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
     globals()[sys.argv[2]](_Var(_lib), *[int(a) if a.lstrip("-").isdigit() else a
