@@ -74,7 +74,10 @@ using namespace rapt;
 struct rapt_batch {
   rapt_ctx* ctx = nullptr;
   int64_t n = 0;
-  double costly = 0.0;  // of the uploaded particles (default_layout)
+  // of the uploaded particles (default_layout): costs in units of the largest,
+  // the largest v / r and output step times v / r, output steps equal
+  double costly = 0.0, v_r = 0.0, row_v_r = 0.0;
+  bool equal_rows = false;
   char* mem = nullptr;  // one allocation for d_state .. d_order and d_work
   double* d_state = nullptr;
   double* d_state0 = nullptr;  // state as uploaded (rapt_batch_reset)
@@ -703,20 +706,30 @@ int rapt_batch_upload(rapt_batch* b, const double* state, const int32_t* flags) 
   for (int64_t i = 1; i < b->n && equal; ++i) equal = dts[i] == dts[0];
   try {
     std::vector<WorkKey> key((size_t)b->n);
+    double v_r = 0.0, row_v_r = 0.0;
     for (int64_t i = 0; i < b->n; ++i) {
-      double k = dts[i];
-      if (equal) {
+      double k = dts[i], cost = 0.0;
+      if (v[i] > 0.0) {  // (a full orbit has no speed here)
         const double *yx = y + i, *yy = yx + b->n, *yz = yy + b->n;
-        k = sqrt(*yx * *yx + *yy * *yy + *yz * *yz) / v[i];
+        const double r = sqrt(*yx * *yx + *yy * *yy + *yz * *yz), rate = v[i] / r;
+        v_r = rate > v_r ? rate : v_r;
+        row_v_r = dts[i] * rate > row_v_r ? dts[i] * rate : row_v_r;
+        cost = rate;
+        if (equal) k = r / v[i];
+      } else if (equal) {
+        k = HUGE_VAL;
       }
       if (!(k > 0.0)) k = HUGE_VAL;  // (no step, no speed, not a number: last)
-      const double cost = 1.0 / k;
+      if (!equal) cost = 1.0 / k;
       sum += cost;
       most = cost > most ? cost : most;
       key[(size_t)i].item = i;
       memcpy(&key[(size_t)i].bits, &k, sizeof k);
     }
     b->costly = costly(b->n, sum, most);
+    b->v_r = v_r;
+    b->row_v_r = row_v_r;
+    b->equal_rows = equal;
     const std::vector<int64_t> order = sorted_items(key);
     HIP_OK(c, hipMemcpyAsync(b->d_order, order.data(), sizeof(int64_t) * b->n,
                              hipMemcpyHostToDevice, c->stream));
@@ -851,7 +864,13 @@ static int spread_lanes(int64_t n, int64_t waves, bool grid) {
 // 6.05, pairs two waves a SIMD 5.39 and 5.70): quads all resident there, and from
 // `one` on the two waves of pairs (131,072 9.1 and 8.8, quads 11.1 and 10.8).
 //
-// Octets that are all resident, one wave a SIMD, need no such thing.  In input
+// Octets that are all resident, one wave a SIMD, need no such thing, but twice
+// the waves of quads start, ask the queue and add to the counters: 8 ns a
+// particle, and a step of the chain is 0.35 us shorter.  `steps` of the longest
+// particle have to make up for it: DoubleDipole electrons, four launches of one and
+// of eight output steps of about 10 steps (quads, octets, ms): 2,048 0.415, 0.435 and
+// 1.76, 1.52; 8,192 0.76, 1.05 and 2.52, 2.58 (32 output steps 7.93, 7.31).
+// In input
 // order the front of the queue is not the costliest, and a gridded field waits
 // for memory, which a second wave hides: quads above that, on a grid above
 // twice that (65,536: 21.8 against 22.6, and 45 against 83 on a grid; octets for
@@ -860,8 +879,9 @@ static int spread_lanes(int64_t n, int64_t waves, bool grid) {
 // and pairs in that order 30.4; 16,384 16.9, octets 10.4).  A uniform field's step
 // is short and a launch's start and end most of it: quads up to `one` / 4 (four
 // rows each, 8,192 0.08, octets 0.13; 24,576 0.19, quads one wave a SIMD 0.14).
+static constexpr double STEPS_R_V = 24.0;  // steps a guiding centre takes in a time r / v
 static void default_layout(const rapt_ctx* c, rapt_trace_desc& d, int64_t n, bool ordered,
-                           double costly) {
+                           double costly, double steps) {
   const int model = c->field.model;
   if (d.mode != RAPT_MODE_GC || d.stepper != RAPT_STEP_DOPRI5 ||
       d.precision != RAPT_PREC_FP64 || d.lanes_per_particle != 0 || d.lanes > 0 ||
@@ -879,10 +899,12 @@ static void default_layout(const rapt_ctx* c, rapt_trace_desc& d, int64_t n, boo
   const int64_t quads = (3 * one / 2 - n) / 8;  // in front of the pairs
   d.lanes_per_particle = 4;
   if (uniform && n <= one / 4) return;
-  if (n <= one / 8 || (ordered && n <= one / 4 && (grid || sheet || costly <= one / 8))) {
+  const bool few = n <= one / 8 ||
+                   (ordered && n <= one / 4 && (grid || sheet || costly <= one / 8));
+  if (few && (grid || 100.0 * steps >= (double)n)) {
     d.lanes_per_particle = 8;
     d.lanes = one;
-  } else if (!ordered || grid || sheet) {
+  } else if (!ordered || grid || sheet || n <= one / 4) {
     return;
   } else if (n <= one / 2 && costly <= one / 4) {
     d.lanes = one;
@@ -898,6 +920,18 @@ static void default_layout(const rapt_ctx* c, rapt_trace_desc& d, int64_t n, boo
     return;
   }
   if (d.block == 0) d.block = 64;
+}
+
+// The layout of a run over the uploaded particles, and of an epoch of it.  The
+// particles of an epoch write the same number of rows: where output steps
+// differ, being a fraction of the bounce period, they cost about the same.
+static void run_layout(const rapt_batch* b, rapt_trace_desc& d) {
+  default_layout(b->ctx, d, b->n, true, b->costly, STEPS_R_V * d.delta * b->v_r);
+}
+static void epoch_layout(const rapt_batch* b, rapt_trace_desc& d, int32_t rows) {
+  const double run = d.delta * b->v_r, epoch = rows * b->row_v_r;
+  default_layout(b->ctx, d, b->n, true, b->equal_rows ? b->costly : (double)b->n,
+                 STEPS_R_V * (epoch < run ? epoch : run));
 }
 
 // Validates a descriptor and builds the kernel arguments of a batch run.
@@ -1122,7 +1156,7 @@ int rapt_batch_run(rapt_batch* b, const rapt_trace_desc* desc, rapt_counters* cn
   rapt_ctx* c = b->ctx;
   rapt_trace_desc dd = *desc;
   const rapt_trace_desc* d = &dd;
-  default_layout(c, dd, b->n, true, b->costly);
+  run_layout(b, dd);
   KArgs A;
   int block = 256;
   int64_t lanes = 0;
@@ -1212,7 +1246,8 @@ int rapt_trace_device_noalloc(rapt_ctx* c, const rapt_trace_desc* d, int64_t n,
   // a user-written field: one lane per particle (compiled if an earlier run
   // loaded that kernel, else interpreted; loading a module allocates)
   if (c->field.model == RAPT_FIELD_EXPR) dd.lanes_per_particle = 1;
-  default_layout(c, dd, n, order != nullptr, (double)n);
+  // (nothing is known of the particles: as if they were alike and the run short)
+  default_layout(c, dd, n, order != nullptr, (double)n, 20.0);
   KArgs A;
   int block = 256;
   int64_t lanes = 0;
@@ -1294,7 +1329,7 @@ int rapt_batch_epochs_begin(rapt_batch* b, const rapt_trace_desc* desc,
   rapt_ctx* c = b->ctx;
   rapt_trace_desc dd = *desc;
   const rapt_trace_desc* d = &dd;
-  default_layout(c, dd, b->n, true, b->costly);
+  epoch_layout(b, dd, rows_per_epoch);
   if (rows_per_epoch < 1) return set_err(c, RAPT_E_ARG, "rows_per_epoch must be >= 1");
   const int width = d->mode == RAPT_MODE_PARTICLE ? 7 : (d->mode == RAPT_MODE_GC ? 5 : 8);
   rapt_batch_epochs_end(b);

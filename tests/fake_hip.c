@@ -23,7 +23,8 @@ size_t fake_overflow_bytes; /* the next copy from the device of this many bytes 
 int fake_pinned_lookup;    /* 1: every host pointer is one of the runtime's */
 int fake_copies;           /* asynchronous copies */
 size_t fake_largest_copy;  /* bytes, of those from the device */
-const char* fake_last_kernel = "";
+const char *fake_last_kernel = "", *fake_epoch_kernel = ""; /* ..., of those captured */
+static int capturing;
 unsigned fake_last_grid, fake_last_block;
 static hipError_t last;
 
@@ -102,6 +103,7 @@ hipError_t hipStreamSynchronize(hipStream_t st) {
 static void launched(const char* name, unsigned grid, unsigned block) {
   ++fake_pending;
   fake_last_kernel = name;
+  if (capturing && strstr(name, "k_trace")) fake_epoch_kernel = name;
   fake_last_grid = grid;
   fake_last_block = block;
 }
@@ -210,11 +212,13 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
 }
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode m) {
   (void)s, (void)m;
+  capturing = 1;
   return hipSuccess;
 }
 hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) {
   static int token;
   (void)s;
+  capturing = 0;
   *g = (hipGraph_t)&token;
   return hipSuccess;
 }

@@ -36,6 +36,17 @@ def _run(fake, case, *args):
     assert r.returncode == 0, r.stderr[-2000:]
 
 
+def _arg(text):
+    try:
+        return int(text)
+    except ValueError:
+        pass
+    try:
+        return float(text)
+    except ValueError:
+        return text
+
+
 class _Grid(F.Grid):
     def parsefile(self, filename):
         a = np.linspace(-8, 8, 9) * rapt.Re
@@ -71,7 +82,7 @@ class _Var:
     def __getattr__(self, name):
         t = {"fake_budget": C.c_size_t, "fake_used": C.c_size_t, "fake_largest_copy": C.c_size_t,
              "fake_overflow_bytes": C.c_size_t, "fake_last_grid": C.c_uint, "fake_last_block": C.c_uint,
-             "fake_last_kernel": C.c_char_p}.get(name, C.c_int)
+             "fake_last_kernel": C.c_char_p, "fake_epoch_kernel": C.c_char_p}.get(name, C.c_int)
         return t.in_dll(self._lib, name)
 
 
@@ -113,13 +124,33 @@ def case_layout(rt, name, n, costs, kernel, lanes):
     b = N.Batch(ctx, n)
     b.upload(S, np.zeros(n, np.int32))
     b.set_rows(5, np.full(n, 1, np.int64))
-    desc = N.make_desc(N.MODE_GC, rapt.params, 1.0)
+    desc = N.make_desc(N.MODE_GC, rapt.params, 10.0)
     for how in ("uploaded", "set_cost"):
         if how == "set_cost":
             b.set_cost(c)
         b.run(desc)
         assert kernel in rt.fake_last_kernel.value.decode(), rt.fake_last_kernel.value
         assert rt.fake_last_grid.value * rt.fake_last_block.value == lanes
+
+
+def case_short(rt, rows, n, v_r, kernel):
+    """Runs and epochs of `rows` output steps of v_r times r / v."""
+    ctx = _ctx(_field("double"))
+    S = np.zeros((N.NSLOT, n))
+    S[N.S_Y0] = 5 * rapt.Re
+    S[N.S_V] = np.linspace(1e8, 0.2e8, n)
+    S[N.S_DT] = v_r * S[N.S_Y0] / S[N.S_V]
+    if n > 1:
+        S[N.S_DT] *= np.linspace(0.999, 1.0, n)  # (output steps that differ)
+    b = N.Batch(ctx, n)
+    b.upload(S, np.zeros(n, np.int32))
+    b.set_rows(5, np.full(n, 1, np.int64))
+    b.run(N.make_desc(N.MODE_GC, rapt.params, rows * v_r * S[N.S_Y0, 0] / 1e8))
+    assert kernel in rt.fake_last_kernel.value.decode(), rt.fake_last_kernel.value
+    if n <= 8192:
+        for _ in b.epochs(N.make_desc(N.MODE_GC, rapt.params, 1e6), rows, 1):
+            pass
+        assert kernel in rt.fake_epoch_kernel.value.decode()
 
 
 _Q, _O, _MIX = "k_trace_gcnILi%dELi4E", "k_trace_gcnILi%dELi8E", "k_trace_gcmixILi%dE"
@@ -139,6 +170,36 @@ ONE = 65536  # lanes of one wave a SIMD
     ("bz", 3, 8192, "equal", _Q, 32768), ("bz", 3, 1, "equal", _Q, 64)])
 def test_default_guiding_centre_layout(fake, name, model, n, costs, kernel, lanes):
     _run(fake, "case_layout", name, n, costs, kernel % model, lanes)
+
+
+@pytest.mark.parametrize("rows,n,v_r,kernel", [
+    (1, 16, 0.4, _O), (1, 4096, 0.4, _Q), (8, 4096, 0.4, _O), (1, 8192, 0.4, _Q),
+    (32, 8192, 0.4, _O), (8, 12000, 0.4, _Q), (16, 12000, 0.4, _O)])
+def test_short_guiding_centre_runs(fake, rows, n, v_r, kernel):
+    """Octets where the steps make up for the launch of twice the waves."""
+    _run(fake, "case_short", rows, n, v_r, kernel % 2)
+
+
+def test_epochs_of_particles_that_cost_the_same(fake):
+    """Output steps of a bounce period's fraction: an epoch's particles cost the
+    same, so all are resident; equal output steps: as they differ in r / v."""
+    _run(fake, "case_epochs")
+
+
+def case_epochs(rt):
+    n = 16384
+    ctx = _ctx(_field("double"))
+    S = np.zeros((N.NSLOT, n))
+    S[N.S_Y0] = 5 * rapt.Re
+    S[N.S_V] = 1e8 * ((np.arange(n) + 1.0) / n) ** 2
+    for dt, kernel in ((0.4 * S[N.S_Y0] / S[N.S_V], _Q % 2), (np.ones(n), _O % 2)):
+        S[N.S_DT] = dt
+        b = N.Batch(ctx, n)
+        b.upload(S, np.zeros(n, np.int32))
+        b.set_rows(5, np.full(n, 1, np.int64))
+        for _ in b.epochs(N.make_desc(N.MODE_GC, rapt.params, 1e9), 32, 1):
+            pass
+        assert kernel in rt.fake_epoch_kernel.value.decode()
 
 
 # ---- full orbits and adaptive runs ---------------------------------------------------
@@ -315,5 +376,4 @@ def test_large_results_to_the_runtimes_own_memory_are_one_copy(fake, known):
 
 if __name__ == "__main__":
     _lib = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
-    globals()[sys.argv[2]](_Var(_lib), *[int(a) if a.lstrip("-").isdigit() else a
-                                         for a in sys.argv[3:]])
+    globals()[sys.argv[2]](_Var(_lib), *[_arg(a) for a in sys.argv[3:]])
