@@ -102,8 +102,7 @@ void k_trace(KArgs A) {
   const int eom = SP ? (int)EOM_TCB : A.eom;
   const FieldC& F = A.F;
   const int64_t n = cold()->n;
-  bool active = false,
-       exhausted = KIND == KIND_ADAPTIVE && (int)(threadIdx.x & 63) >= cold()->wave_lanes;
+  bool active = false, exhausted = false;
   int64_t pi = 0;
   // per-lane particle + integrator state
   double x = 0, y[6] = {0, 0, 0, 0, 0, 0}, k1[6] = {0, 0, 0, 0, 0, 0};
@@ -193,7 +192,11 @@ void k_trace(KArgs A) {
   for (;;) {
     // ---- refill: take the next particle ---------------------------------------
     if (!active && !exhausted) {
-      pi = (int64_t)atomicAdd(&cold()->work[0], 1ULL);
+      // (a spread run's idle lanes find the queue empty; decided here and not in
+      // front of the loop, where it made one lane's run up to 7% longer)
+      pi = n;
+      if (KIND != KIND_ADAPTIVE || (int)(threadIdx.x & 63) < cold()->wave_lanes)
+        pi = (int64_t)atomicAdd(&cold()->work[0], 1ULL);
       if (pi < n && cold()->order) pi = cold()->order[pi];
       if (pi >= n) {
         exhausted = true;

@@ -78,6 +78,7 @@ struct rapt_batch {
   // the largest v / r and output step times v / r, output steps equal
   double costly = 0.0, v_r = 0.0, row_v_r = 0.0;
   bool equal_rows = false;
+  int64_t max_cap = 0;  // the largest row capacity
   char* mem = nullptr;  // one allocation for d_state .. d_order and d_work
   double* d_state = nullptr;
   double* d_state0 = nullptr;  // state as uploaded (rapt_batch_reset)
@@ -781,7 +782,7 @@ int rapt_batch_set_rows(rapt_batch* b, int32_t width, const int64_t* row_cap) {
   HIP_OK(c, hipSetDevice(c->device));
   int64_t* off = (int64_t*)malloc(sizeof(int64_t) * b->n);
   if (!off) return set_err(c, RAPT_E_OOM, "host allocation failed");
-  int64_t tot = 0;
+  int64_t tot = 0, most = 0;
   for (int64_t i = 0; i < b->n; ++i) {
     if (row_cap[i] < 0) {
       free(off);
@@ -789,6 +790,7 @@ int rapt_batch_set_rows(rapt_batch* b, int32_t width, const int64_t* row_cap) {
     }
     off[i] = tot;
     tot += row_cap[i];
+    most = row_cap[i] > most ? row_cap[i] : most;
   }
   if (tot * width != b->total_rows * b->width || !b->d_rows) {
     (void)hipFree(b->d_rows);
@@ -802,6 +804,7 @@ int rapt_batch_set_rows(rapt_batch* b, int32_t width, const int64_t* row_cap) {
   }
   b->total_rows = tot;
   b->width = width;
+  b->max_cap = most;
   hipError_t e1 = hipMemcpyAsync(b->d_rowoff, off, sizeof(int64_t) * b->n,
                                  hipMemcpyHostToDevice, c->stream);
   hipError_t e2 = hipMemcpyAsync(b->d_rowcap, row_cap, sizeof(int64_t) * b->n,
@@ -815,26 +818,40 @@ int rapt_batch_set_rows(rapt_batch* b, int32_t width, const int64_t* row_cap) {
 
 }  // extern "C"
 
-// Lanes of a wave that take particles in an ADAPTIVE run: as few as leave
-// `waves` waves for the launch, a power of two.  A wave's step runs every path
-// that any of its particles takes, here a full-orbit step, a guiding-centre step,
-// an adiabaticity test and a conversion, so a launch that does not fill the GPU
-// is faster with its particles spread over more waves, up to one a SIMD
-// (current-sheet protons, spread so and packed: 100 3.7 and 7.9 ms, 500 4.3 and
-// 9.1, 4,096 7.5 and 9.6, 32,768 8.7 and 9.3; with two waves a SIMD 4,096 take
-// 8.1 and 32,768 11.3).  A gridded field waits for memory, and the waves of fewer
-// particles each ask for more of it: there only particles that get a wave of
-// their own are spread (256 on a grid of three times 7.4 and 9.1, 1,000 10.4
-// and 11.2; with several a wave 8,192 7.1 and 6.5, 16,384 7.2 and 6.7).
-// Full-orbit and guiding-centre runs take one path and are not: 4,096 protons
+// Lanes of a wave that take particles in an ADAPTIVE run whose particles write
+// about `rows` rows, a power of two.  A wave's step runs every path that any of its
+// particles takes, here a full-orbit step, a guiding-centre step, an adiabaticity
+// test and a conversion, so fewer particles a wave take less; but waves of one CU
+// in different places of the kernel share its instruction cache (some 100 KB run
+// each step), which costs about as much where the waves still hold several
+// particles, and more waves take longer to start.  Kernel time, ms: 64 a wave, one
+// wave a CU (256), one a SIMD (1,024):
+//   500 sheet protons, advance(30)                      8.7, 4.8, 4.6
+//   1,024 in the dipole, advance(2)                     1.65, 1.26, 1.01
+//   the same, advance(0.02), about two rows             0.175, 0.163, 0.180
+//   2,048 in the sheet, advance(10), GCtimestep 0.1     4.2, 3.9, 4.9
+//   4,096 in the sheet, advance(30) / that              9.1, 7.6, 7.7 / 4.1, 4.0, 5.3
+//   8,192 / the same                                    9.3, 9.2, 8.9 / 3.8, 4.2, 5.7
+//   16,384 / the same                                   9.1, 9.3, 7.7 / 3.9, 3.9, 3.6
+//   16,384 in the dipole, advance(0.02)                 0.181, 0.179, 0.218
+//   1,024 on a grid, advance(0.3)                       4.6, 4.0, 4.5
+// So: a wave each up to one a SIMD (on a grid, whose waves wait for memory, and for
+// a row or two up to one a CU), one wave a CU up to 16 particles each, and from 64
+// a CU on, where rows are many, one a SIMD again.
+// Full-orbit and guiding-centre runs take one path and are not spread: 4,096 protons
 // 6.3 ms packed and 7.6 spread, 1,000 guiding centres on octets 5.0 and 6.3.
-static constexpr int SPREAD_WAVES = 4;  // waves a CU: one a SIMD
-static int spread_lanes(int64_t n, int64_t waves, bool grid) {
-  if (grid) return n <= waves ? 1 : 64;
+static int spread_lanes(int64_t n, int64_t rows, int cus, bool grid) {
+  int64_t waves = cus;
+  if (!grid && ((n <= 4 * cus && rows >= 3) || (n >= 64 * cus && rows >= 8)))
+    waves = 4 * cus;
+  else if (n > 16 * cus)
+    return 64;
   int wl = 64;
   while (wl > 1 && (n + wl / 2 - 1) / (wl / 2) <= waves) wl /= 2;
   return wl;
 }
+// Rows that advance_adaptive (batch.py) has room for beside those it expects
+static constexpr int64_t SPARE_ROWS = 11;
 
 // The layout of a guiding-centre run with lanes_per_particle 0 and lanes 0.  A
 // lone wave issues an instruction in nearly every slot of its SIMD, so what
@@ -934,8 +951,9 @@ static void epoch_layout(const rapt_batch* b, rapt_trace_desc& d, int32_t rows) 
                  STEPS_R_V * (epoch < run ? epoch : run));
 }
 
-// Validates a descriptor and builds the kernel arguments of a batch run.
-static int prepare_run(rapt_batch* b, const rapt_trace_desc* d, KArgs& A, int& block_out,
+// Validates a descriptor and builds the kernel arguments of a batch run, whose
+// particles write about `rows` rows (0: not known).
+static int prepare_run(rapt_batch* b, const rapt_trace_desc* d, int64_t rows, KArgs& A, int& block_out,
                        int64_t& lanes_out, bool& grouped_out) {
   if (!b || !d) return RAPT_E_ARG;
   rapt_ctx* c = b->ctx;
@@ -1066,8 +1084,7 @@ static int prepare_run(rapt_batch* b, const rapt_trace_desc* d, KArgs& A, int& b
   int block = d->block > 0 ? d->block : 0;
   A.wave_lanes = 64;
   if (d->mode == RAPT_MODE_ADAPTIVE && d->lanes <= 0) {
-    A.wave_lanes = spread_lanes(b->n, (int64_t)SPREAD_WAVES * cus,
-                                c->field.model == RAPT_FIELD_GRID);
+    A.wave_lanes = spread_lanes(b->n, rows, cus, c->field.model == RAPT_FIELD_GRID);
     lanes = (b->n + A.wave_lanes - 1) / A.wave_lanes * 64;
   }
   if (block == 0) {
@@ -1161,7 +1178,7 @@ int rapt_batch_run(rapt_batch* b, const rapt_trace_desc* desc, rapt_counters* cn
   int block = 256;
   int64_t lanes = 0;
   bool grouped = false;
-  int rc = prepare_run(b, d, A, block, lanes, grouped);
+  int rc = prepare_run(b, d, b->max_cap - SPARE_ROWS, A, block, lanes, grouped);
   if (!rc) rc = prepare_jit(c, d, A, grouped);
   if (rc) return rc;
   HIP_OK(c, hipMemsetAsync(b->d_work, 0, sizeof(unsigned long long) * 8, c->stream));
@@ -1252,7 +1269,7 @@ int rapt_trace_device_noalloc(rapt_ctx* c, const rapt_trace_desc* d, int64_t n,
   int block = 256;
   int64_t lanes = 0;
   bool grouped = false;
-  const int rc = prepare_run(&view, &dd, A, block, lanes, grouped);
+  const int rc = prepare_run(&view, &dd, 0, A, block, lanes, grouped);
   if (rc) return rc;
   // the scratch keeps the last call's counters: clear them
   hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, c->stream, c->noalloc_scratch,
@@ -1363,7 +1380,7 @@ int rapt_batch_epochs_begin(rapt_batch* b, const rapt_trace_desc* desc,
   int block = 256;
   int64_t lanes = 0;
   bool grouped = false;
-  int rc = prepare_run(b, d, A, block, lanes, grouped);
+  int rc = prepare_run(b, d, rows_per_epoch, A, block, lanes, grouped);
   b->width = w0;
   if (!rc) rc = prepare_jit(c, d, A, grouped);  // before the capture: loading allocates
   if (rc) {

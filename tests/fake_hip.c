@@ -25,7 +25,7 @@ int fake_copies;           /* asynchronous copies */
 size_t fake_largest_copy;  /* bytes, of those from the device */
 const char *fake_last_kernel = "", *fake_epoch_kernel = ""; /* ..., of those captured */
 static int capturing;
-unsigned fake_last_grid, fake_last_block;
+unsigned fake_last_grid, fake_last_block, fake_epoch_lanes;
 static hipError_t last;
 
 static hipError_t ret(hipError_t e) {
@@ -103,7 +103,10 @@ hipError_t hipStreamSynchronize(hipStream_t st) {
 static void launched(const char* name, unsigned grid, unsigned block) {
   ++fake_pending;
   fake_last_kernel = name;
-  if (capturing && strstr(name, "k_trace")) fake_epoch_kernel = name;
+  if (capturing && strstr(name, "k_trace")) {
+    fake_epoch_kernel = name;
+    fake_epoch_lanes = grid * block;
+  }
   fake_last_grid = grid;
   fake_last_block = block;
 }

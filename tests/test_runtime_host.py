@@ -82,6 +82,7 @@ class _Var:
     def __getattr__(self, name):
         t = {"fake_budget": C.c_size_t, "fake_used": C.c_size_t, "fake_largest_copy": C.c_size_t,
              "fake_overflow_bytes": C.c_size_t, "fake_last_grid": C.c_uint, "fake_last_block": C.c_uint,
+             "fake_epoch_lanes": C.c_uint,
              "fake_last_kernel": C.c_char_p, "fake_epoch_kernel": C.c_char_p}.get(name, C.c_int)
         return t.in_dll(self._lib, name)
 
@@ -205,30 +206,42 @@ def case_epochs(rt):
 # ---- full orbits and adaptive runs ---------------------------------------------------
 
 
-def case_orbits(rt, name, mode, n, kernel, waves):
+def case_orbits(rt, name, mode, n, rows, kernel, waves):
     ctx = _ctx(_field(name))
     S = np.zeros((N.NSLOT, n))
     S[N.S_Y0] = 5 * rapt.Re
     b = N.Batch(ctx, n)
     b.upload(S, np.zeros(n, np.int32))
-    b.set_rows(N.ROW_WIDTH[mode], np.full(n, 1, np.int64))
-    b.run(N.make_desc(mode, dict(rapt.params, GCtimestep=0.1), 1.0))
+    b.set_rows(N.ROW_WIDTH[mode], np.full(n, rows + 11, np.int64))
+    desc = N.make_desc(mode, dict(rapt.params, GCtimestep=0.1), 1.0)
+    b.run(desc)
     assert kernel in rt.fake_last_kernel.value.decode(), rt.fake_last_kernel.value
     assert rt.fake_last_grid.value * rt.fake_last_block.value == 64 * waves
+    if mode == N.MODE_ADAPTIVE:
+        for _ in b.epochs(desc, rows, 1):
+            pass
+        assert kernel in rt.fake_epoch_kernel.value.decode()
+        assert rt.fake_epoch_lanes.value == 64 * waves
 
 
 _P, _A = N.MODE_PARTICLE, N.MODE_ADAPTIVE
+_DIP, _GRID = "ILi1ELi2ELi0ELb1E", "ILi9ELi2ELi0ELb0E"
 
 
-@pytest.mark.parametrize("name,mode,n,kernel,waves", [
+@pytest.mark.parametrize("name,mode,n,rows,kernel,waves", [
     # the static kernel where it is the faster one
-    ("dipole", _P, 1024, "ILi1ELi0ELi0ELb1E", 16), ("grid", _P, 1024, "ILi9ELi0ELi0ELb0E", 16),
-    ("dipole", _A, 4096, "ILi1ELi2ELi0ELb1E", 1024), ("user", _P, 64, "ILi10ELi0ELi0ELb0E", 1),
-    # on a grid, a wave each or 64 a wave
-    ("grid", _A, 1, "ILi9ELi2ELi0ELb0E", 1), ("grid", _A, 1024, "ILi9ELi2ELi0ELb0E", 1024),
-    ("grid", _A, 1025, "ILi9ELi2ELi0ELb0E", 17), ("grid", _A, 16384, "ILi9ELi2ELi0ELb0E", 256)])
-def test_orbit_kernels_and_spread(fake, name, mode, n, kernel, waves):
-    _run(fake, "case_orbits", name, mode, n, kernel, waves)
+    ("dipole", _P, 1024, 9, "ILi1ELi0ELi0ELb1E", 16),
+    ("grid", _P, 1024, 9, "ILi9ELi0ELi0ELb0E", 16), ("user", _P, 64, 9, "ILi10ELi0ELi0ELb0E", 1),
+    # a wave each, one wave a CU, 64 a wave, one wave a SIMD
+    ("dipole", _A, 1, 1, _DIP, 1), ("dipole", _A, 256, 1, _DIP, 256),
+    ("dipole", _A, 1024, 3, _DIP, 1024), ("dipole", _A, 1024, 2, _DIP, 256),
+    ("dipole", _A, 1025, 99, _DIP, 129), ("dipole", _A, 4096, 99, _DIP, 256),
+    ("dipole", _A, 4097, 99, _DIP, 65), ("dipole", _A, 16383, 99, _DIP, 256),
+    ("dipole", _A, 16384, 8, _DIP, 1024), ("dipole", _A, 16384, 7, _DIP, 256),
+    ("grid", _A, 1, 99, _GRID, 1), ("grid", _A, 1024, 99, _GRID, 256),
+    ("grid", _A, 4096, 99, _GRID, 256), ("grid", _A, 16384, 99, _GRID, 256)])
+def test_orbit_kernels_and_spread(fake, name, mode, n, rows, kernel, waves):
+    _run(fake, "case_orbits", name, mode, n, rows, kernel, waves)
 
 
 # ---- kept scratch --------------------------------------------------------------------
