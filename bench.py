@@ -868,6 +868,9 @@ def run_surrogate(args):
     res["ms_per_step"] = (kms / 1e3 + idx.size / traced_rate) * 1e3
     res["traced_queries_per_s"] = traced_rate
     res["speedup_vs_traced"] = value / traced_rate
+    res["traced_note"] = ("the traced labels of a dipole-type field run on 72 of 2,048 waves "
+                          "(rapt_bounce.hip); with every wave 65,536 take 5.2 ms, 1.3e7 "
+                          "queries/s, and the gain is about 90")
     res["inference_kernel_ms"] = kms
     res["inference_wall_ms"] = t_inf * 1e3
     res["fallback_queries"] = int(idx.size)

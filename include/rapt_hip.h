@@ -110,13 +110,15 @@ typedef struct {
                                     work order on lane quads, the rest on lane pairs;
                                     5 = mixed: the first mixed_octets on octets, the
                                     next mixed_quads on quads, the rest on pairs;
-                                    0 (default) = by the number of particles, with the
-                                    resident lanes (quads where lanes is given).
+                                    0 (default) = by the number of particles, what the
+                                    run is expected to cost them and the field, with
+                                    the resident lanes (quads where lanes is given).
                                     Results do not depend on it */
     int32_t work_order;          /* 0: the batch's queue order (shortest output step
-                                    first, or by cost after rapt_batch_set_cost); 1:
-                                    input order.  Results per particle do not depend
-                                    on it */
+                                    first; where all output steps are equal, shortest
+                                    distance from the origin over speed first; or by
+                                    cost after rapt_batch_set_cost); 1: input order.
+                                    Results per particle do not depend on it */
     int64_t mixed_quads;         /* lanes_per_particle 3, 5: particles on quads (0: n/8) */
     int64_t mixed_octets;        /* lanes_per_particle 5: particles on octets (0: n/64) */
 } rapt_trace_desc;

@@ -231,6 +231,7 @@ def advance_adaptive(field, pos, vel, t0, mass, charge, delta, params=None, row_
     if row_cap is None:
         dtp = particle_dt(field, last7, mass, charge, P["cyclotronresolution"], device)
         gcdt = float(P.get("GCtimestep", 0.0)) or 1.0
+        # (eleven rows to spare, as rapt_tracer.hip's SPARE_ROWS has them)
         row_cap = _rows_needed(delta, np.minimum(dtp, gcdt)) + 8
     desc = N.make_desc(N.MODE_ADAPTIVE, P, delta, lanes=lanes, **kw)
     return _run(field, N.MODE_ADAPTIVE, S, flags, row_cap, desc, device)

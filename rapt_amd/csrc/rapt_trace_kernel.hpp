@@ -85,8 +85,9 @@ struct GcRHS {
 // and a square root, 32 instructions of ~95) and its reciprocal in every stage
 // and throws them away in a static field.
 // Register budget: two waves per SIMD (256 registers per lane) for the
-// analytic fields, where it costs 12-92 bytes of spills per lane in the GC
-// and Particle kernels and hides the dependent-chain latency better (one-lane
+// analytic fields, where it costs 0-148 bytes of spills per lane in the Particle
+// kernels, 36-320 in the one-lane GC ones and 76-516 in the adaptive ones and
+// hides the dependent-chain latency better (one-lane
 // GC +21% FP64, +31% FP32-field on 1,048,576 particles); one wave for
 // gridded fields, where two spill 180 bytes per lane in the Particle kernel
 // and ran 15% slower (65,536 protons in a 257 x 257 x 193 dipole grid), and

@@ -251,7 +251,8 @@ static void launch_trace(rapt_ctx* c, const KArgs& A, int block, int64_t lanes) 
 template <int K>
 static void launch_model(rapt_ctx* c, const KArgs& A, int block, int64_t lanes) {
   // a compiled user-written field, once its kernel is loaded (otherwise the
-  // built-in kernel interprets the program: the same results)
+  // built-in kernel interprets the program: the same results); its full-orbit and
+  // adaptive kernels are the general ones, static field or not
   if (c->field.model == RAPT_FIELD_EXPR && c->expr_mode == RAPT_EXPR_COMPILED &&
       rapt_jit_launch(c, K, K == KIND_GC && trace_use_sp<F_EXPR>(A), A, block, lanes))
     return;
