@@ -147,6 +147,40 @@ static double costly(int64_t n, double sum, double most) {
   return k >= 1.0 && k <= (double)n ? k : (double)n;
 }
 
+// What the layouts of a run and an epoch go by, from the sorted keys of the work
+// order and the state; some 4,096 particles stand for a larger batch (65,536:
+// 0.05 ms, every one 0.25).
+static void expect_costs(rapt_batch* b, const std::vector<WorkKey>& key, const double* state,
+                         bool equal) {
+  const int64_t n = b->n;
+  auto at = [&key](int64_t j) {
+    double k;
+    memcpy(&k, &key[(size_t)j].bits, sizeof k);
+    return k;
+  };
+  const int64_t step = (n + 4095) / 4096;
+  double sum = 0.0, m = 0.0;
+  for (int64_t j = step / 2; j < n; j += step, m += 1.0) sum += 1.0 / at(j);
+  b->costly = costly(n, sum / m * (double)n, 1.0 / at(0));
+  b->equal_rows = equal;
+  const double* dts = state + (size_t)RAPT_S_DT * n;
+  if (equal) {
+    b->v_r = 1.0 / at(0);
+    b->row_v_r = dts[0] * b->v_r;
+    return;
+  }
+  const double* v = state + (size_t)RAPT_S_V * n;
+  const double* y = state + (size_t)RAPT_S_Y0 * n;
+  b->v_r = b->row_v_r = 0.0;
+  for (int64_t i = 0; i < n; i += n / 4096 | 1) {
+    if (!(v[i] > 0.0)) continue;  // (a full orbit has no speed here)
+    const double *yx = y + i, *yy = yx + n, *yz = yy + n;
+    const double rate = v[i] / sqrt(*yx * *yx + *yy * *yy + *yz * *yz);
+    b->v_r = rate > b->v_r ? rate : b->v_r;
+    b->row_v_r = dts[i] * rate > b->row_v_r ? dts[i] * rate : b->row_v_r;
+  }
+}
+
 static int field_width(int what) {
   switch (what) {
     case 0: case 1: case 2: case 4: case 7: case 9: return 3;
@@ -703,36 +737,22 @@ int rapt_batch_upload(rapt_batch* b, const double* state, const int32_t* flags) 
   const double* dts = state + (size_t)RAPT_S_DT * b->n;
   const double* v = state + (size_t)RAPT_S_V * b->n;
   const double* y = state + (size_t)RAPT_S_Y0 * b->n;
-  double sum = 0.0, most = 0.0;  // of the steps that the particles may need
   bool equal = dts[0] > 0.0;
   for (int64_t i = 1; i < b->n && equal; ++i) equal = dts[i] == dts[0];
   try {
     std::vector<WorkKey> key((size_t)b->n);
-    double v_r = 0.0, row_v_r = 0.0;
     for (int64_t i = 0; i < b->n; ++i) {
-      double k = dts[i], cost = 0.0;
-      if (v[i] > 0.0) {  // (a full orbit has no speed here)
+      double k = dts[i];
+      if (equal) {
         const double *yx = y + i, *yy = yx + b->n, *yz = yy + b->n;
-        const double r = sqrt(*yx * *yx + *yy * *yy + *yz * *yz), rate = v[i] / r;
-        v_r = rate > v_r ? rate : v_r;
-        row_v_r = dts[i] * rate > row_v_r ? dts[i] * rate : row_v_r;
-        cost = rate;
-        if (equal) k = r / v[i];
-      } else if (equal) {
-        k = HUGE_VAL;
+        k = sqrt(*yx * *yx + *yy * *yy + *yz * *yz) / v[i];
       }
       if (!(k > 0.0)) k = HUGE_VAL;  // (no step, no speed, not a number: last)
-      if (!equal) cost = 1.0 / k;
-      sum += cost;
-      most = cost > most ? cost : most;
       key[(size_t)i].item = i;
       memcpy(&key[(size_t)i].bits, &k, sizeof k);
     }
-    b->costly = costly(b->n, sum, most);
-    b->v_r = v_r;
-    b->row_v_r = row_v_r;
-    b->equal_rows = equal;
     const std::vector<int64_t> order = sorted_items(key);
+    expect_costs(b, key, state, equal);
     HIP_OK(c, hipMemcpyAsync(b->d_order, order.data(), sizeof(int64_t) * b->n,
                              hipMemcpyHostToDevice, c->stream));
     HIP_OK(c, hipStreamSynchronize(c->stream));
@@ -880,23 +900,31 @@ static constexpr int64_t SPARE_ROWS = 11;
 // quads all resident 1.89 and 2.70; 32,768 quads one wave a SIMD 3.45 and 3.72, all
 // resident 3.17 and 3.91; 65,536 quads and pairs 7.15 and 6.33, quads 6.01 and
 // 6.05, pairs two waves a SIMD 5.39 and 5.70): quads all resident there, and from
-// `one` on the two waves of pairs (131,072 9.1 and 8.8, quads 11.1 and 10.8).
+// `one` on the two waves of pairs (131,072 9.1 and 8.8, quads 11.1 and 10.8).  Where
+// costs differ the queue may be a little longer (32,768 of one energy: 1.18 times
+// the resident quads' costliest, 3.73 against 4.08 all resident).
 //
 // Octets that are all resident, one wave a SIMD, need no such thing, but twice
 // the waves of quads start, ask the queue and add to the counters: 8 ns a
 // particle, and a step of the chain is 0.35 us shorter.  `steps` of the longest
-// particle have to make up for it: DoubleDipole electrons, four launches of one and
-// of eight output steps of about 10 steps (quads, octets, ms): 2,048 0.415, 0.435 and
-// 1.76, 1.52; 8,192 0.76, 1.05 and 2.52, 2.58 (32 output steps 7.93, 7.31).
-// In input
-// order the front of the queue is not the costliest, and a gridded field waits
-// for memory, which a second wave hides: quads above that, on a grid above
-// twice that (65,536: 21.8 against 22.6, and 45 against 83 on a grid; octets for
-// few: 8,192 10.0, 8.2; a grid's 16,384 29.9, 23.1).  So too in the current sheet and the
-// parabolic field, whose costs are not r / v's (65,536 in the sheet 19.3, quads
-// and pairs in that order 30.4; 16,384 16.9, octets 10.4).  A uniform field's step
-// is short and a launch's start and end most of it: quads up to `one` / 4 (four
-// rows each, 8,192 0.08, octets 0.13; 24,576 0.19, quads one wave a SIMD 0.14).
+// particle have to make up for it, from about 1,000 particles on: DoubleDipole
+// electrons, four launches of one and of eight output steps of about 10 steps
+// (quads, octets, ms): 1,000 0.403, 0.369 and 1.72, 1.45; 2,048 0.415, 0.435 and
+// 1.76, 1.52; 8,192 0.76, 1.05 and 2.52, 2.58 (32 output steps 7.93, 7.31); in the
+// varying dipole 4,096 0.76, 0.78 and 3.60, 2.96.  Short launches are also
+// the better for a queue worked off in rounds than for a second wave a SIMD
+// (advance(0.02) of 32,768 alike, quads one wave a SIMD 0.33, all resident 0.41).
+//
+// In input order the front of the queue is not the costliest, and a gridded field
+// waits for memory, which a second wave hides: quads above `one` / 8, on a grid
+// above `one` / 4 (65,536: 21.8 against 22.6, and 45 against 83 on a grid; octets for
+// few: 8,192 10.0, 8.2; a grid's 16,384 29.9, 23.1).  In the current sheet and the
+// parabolic field, whose costs are not r / v's, octets and quads as long as they
+// last, one wave a SIMD, and quads all resident above (protons in the sheet: 16,384
+// quads 16.9, octets 10.4; 32,768 alike 9.2, one wave a SIMD 7.2; 65,536 19.3, quads
+// and pairs 30.4).  A uniform field's step is short and a launch's start and end
+// most of it: quads up to `one` / 4 (four rows each, 8,192 0.08, octets 0.13;
+// 24,576 0.19, quads one wave a SIMD 0.14).
 static constexpr double STEPS_R_V = 24.0;  // steps a guiding centre takes in a time r / v
 static void default_layout(const rapt_ctx* c, rapt_trace_desc& d, int64_t n, bool ordered,
                            double costly, double steps) {
@@ -917,16 +945,23 @@ static void default_layout(const rapt_ctx* c, rapt_trace_desc& d, int64_t n, boo
   const int64_t quads = (3 * one / 2 - n) / 8;  // in front of the pairs
   d.lanes_per_particle = 4;
   if (uniform && n <= one / 4) return;
+  // (a step in a field that changes in time takes twice as long)
+  const bool lasting = c->field.is_static == 0;
+  const bool brief = costly >= 0.0 && steps < (lasting ? 50.0 : 100.0);
+  if (costly < 0.0) costly = (double)n;  // not known: as if they were alike
+  // particles of different cost fill the ends of the rounds
+  const double rounds = costly / (1.5 - 0.5 * costly / (double)n);
   const bool few = n <= one / 8 ||
                    (ordered && n <= one / 4 && (grid || sheet || costly <= one / 8));
-  if (few && (grid || 100.0 * steps >= (double)n)) {
+  const double worth = lasting ? 2000.0 + 250.0 * steps : 1000.0 + 150.0 * steps;
+  if (few && (grid || sheet || (double)n <= worth)) {
     d.lanes_per_particle = 8;
     d.lanes = one;
-  } else if (!ordered || grid || sheet || n <= one / 4) {
+  } else if (!ordered || grid || n <= one / 4 || (sheet && n > one / 2)) {
     return;
-  } else if (n <= one / 2 && costly <= one / 4) {
+  } else if (n <= one / 2 && (brief || sheet || rounds <= one / 4)) {
     d.lanes = one;
-  } else if (n > one / 2 && quads > 0 && costly <= one / 2 - quads) {
+  } else if (n > one / 2 && quads > 0 && (brief || rounds <= one / 2 - quads)) {
     d.lanes_per_particle = 3;
     d.mixed_quads = quads;
     d.lanes = one;
@@ -942,14 +977,18 @@ static void default_layout(const rapt_ctx* c, rapt_trace_desc& d, int64_t n, boo
 
 // The layout of a run over the uploaded particles, and of an epoch of it.  The
 // particles of an epoch write the same number of rows: where output steps
-// differ, being a fraction of the bounce period, they cost about the same.
+// differ, being a fraction of the bounce period, they cost about the same, and
+// there are more that take long: as if each step were 2/3 of one.
 static void run_layout(const rapt_batch* b, rapt_trace_desc& d) {
   default_layout(b->ctx, d, b->n, true, b->costly, STEPS_R_V * d.delta * b->v_r);
 }
 static void epoch_layout(const rapt_batch* b, rapt_trace_desc& d, int32_t rows) {
   const double run = d.delta * b->v_r, epoch = rows * b->row_v_r;
-  default_layout(b->ctx, d, b->n, true, b->equal_rows ? b->costly : (double)b->n,
-                 STEPS_R_V * (epoch < run ? epoch : run));
+  const double steps = STEPS_R_V * (epoch < run ? epoch : run);
+  if (b->equal_rows)
+    default_layout(b->ctx, d, b->n, true, b->costly, steps);
+  else
+    default_layout(b->ctx, d, b->n, true, (double)b->n, steps * (2.0 / 3.0));
 }
 
 // Validates a descriptor and builds the kernel arguments of a batch run, whose
@@ -1264,8 +1303,7 @@ int rapt_trace_device_noalloc(rapt_ctx* c, const rapt_trace_desc* d, int64_t n,
   // a user-written field: one lane per particle (compiled if an earlier run
   // loaded that kernel, else interpreted; loading a module allocates)
   if (c->field.model == RAPT_FIELD_EXPR) dd.lanes_per_particle = 1;
-  // (nothing is known of the particles: as if they were alike and the run short)
-  default_layout(c, dd, n, order != nullptr, (double)n, 20.0);
+  default_layout(c, dd, n, order != nullptr, -1.0, 7.0);  // (nothing known: few steps)
   KArgs A;
   int block = 256;
   int64_t lanes = 0;

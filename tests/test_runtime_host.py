@@ -167,7 +167,8 @@ ONE = 65536  # lanes of one wave a SIMD
     ("double", 2, 16384, "spread", _O, ONE), ("double", 2, 32768, "spread", _Q, ONE),
     ("double", 2, 65536, "spread", _MIX, ONE), ("grid", 9, 16384, "equal", _O, ONE),
     # fields that the order says nothing of, or with short steps
-    ("sheet", 7, 40000, "spread", _Q, 160000), ("sheet", 7, 131072, "spread", _Q, 8 * ONE),
+    ("sheet", 7, 32768, "equal", _Q, ONE), ("sheet", 7, 40000, "spread", _Q, 160000),
+    ("sheet", 7, 131072, "spread", _Q, 8 * ONE),
     ("bz", 3, 8192, "equal", _Q, 32768), ("bz", 3, 1, "equal", _Q, 64)])
 def test_default_guiding_centre_layout(fake, name, model, n, costs, kernel, lanes):
     _run(fake, "case_layout", name, n, costs, kernel % model, lanes)
@@ -175,10 +176,31 @@ def test_default_guiding_centre_layout(fake, name, model, n, costs, kernel, lane
 
 @pytest.mark.parametrize("rows,n,v_r,kernel", [
     (1, 16, 0.4, _O), (1, 4096, 0.4, _Q), (8, 4096, 0.4, _O), (1, 8192, 0.4, _Q),
-    (32, 8192, 0.4, _O), (8, 12000, 0.4, _Q), (16, 12000, 0.4, _O)])
+    (32, 8192, 0.4, _O), (4, 12000, 0.4, _Q), (16, 12000, 0.4, _O)])
 def test_short_guiding_centre_runs(fake, rows, n, v_r, kernel):
     """Octets where the steps make up for the launch of twice the waves."""
     _run(fake, "case_short", rows, n, v_r, kernel % 2)
+
+
+def case_brief(rt, n, kernel, lanes):
+    """Particles alike, a run of few steps: one wave a SIMD, in rounds."""
+    ctx = _ctx(_field("double"))
+    S = np.zeros((N.NSLOT, n))
+    S[N.S_Y0] = 5 * rapt.Re
+    S[N.S_V] = 1e8
+    S[N.S_DT] = 0.1
+    b = N.Batch(ctx, n)
+    b.upload(S, np.zeros(n, np.int32))
+    b.set_rows(5, np.full(n, 1, np.int64))
+    b.run(N.make_desc(N.MODE_GC, rapt.params, 0.3))
+    assert kernel in rt.fake_last_kernel.value.decode()
+    assert rt.fake_last_grid.value * rt.fake_last_block.value == lanes
+
+
+@pytest.mark.parametrize("n,kernel,lanes", [(16385, _Q, ONE), (32768, _Q, ONE),
+                                            (65536, _MIX, ONE)])
+def test_brief_runs_of_particles_alike(fake, n, kernel, lanes):
+    _run(fake, "case_brief", n, kernel % 2, lanes)
 
 
 def test_epochs_of_particles_that_cost_the_same(fake):
